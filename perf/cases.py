@@ -279,7 +279,7 @@ def work(case):
         pts = case["nx"] * case["ny"] * case["nz"]
         return {"bytes": 8.0 * 10 * pts, "flops": 230.0 * pts}
     ns, nst, mix = {"duct": (9, 21, 1), "box": (9, 21, 1), "duct_lewis": (9, 21, 0), "methane": (16, 35, 1),
-                    "methane4": (7, 4, 0), "onestep": (2, 1, 0), "batch": (9, 21, 1)}[case["kind"]]
+                    "methane4": (8, 4, 0), "onestep": (2, 1, 0), "batch": (9, 21, 1)}[case["kind"]]
     pts = float(sum(a * b * c for a, b, c in _grids(case)))
     sub = 5.0 * case["steps"] * pts
     stencil = 3.0 * (330.0 + 90.0 * ns) + 500.0
