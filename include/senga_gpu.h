@@ -286,12 +286,11 @@ int sg_memory(sg_handle *h, size_t *bytes);
 int sg_mechanism_compiled(const sg_handle *h, int *compiled);
 
 /* ---- Tiles and their autotuner (no counterpart in the reference) ---------
- * narrow[d] selects the tile of the direction-d derivative pass: 0 = rows of
- * 32 points (default), 1 = rows of 16 points and twice the rows (no idle
- * lanes when n_x is an odd multiple of 16, a shorter halo along y and z).
- * No choice changes any result.  sg_autotune times each choice on the
- * handle's current state (reps launches each, 5 if reps <= 0), keeps the
- * fastest, and returns in *ms the tuned passes' time per substage; the state
+ * The derivative passes have one tile shape (16 x 16 points, see k_pass), so
+ * there is nothing left to choose: narrow[d] (0 or 1, kept for callers that
+ * set it) is stored and returned and changes neither results nor speed.
+ * sg_autotune times the passes on the handle's current state (reps launches
+ * each, 5 if reps <= 0) and returns in *ms their time per substage; the state
  * it leaves is the one it found, so tuned and untuned runs compute identical
  * results. */
 int sg_set_tiles(sg_handle *h, const int narrow[3]);
@@ -337,8 +336,7 @@ int sg_batch_step(sg_batch *b, int nsteps);
  * the failing member's index in *failed (else -1), whose sg_last_error holds
  * the point. */
 int sg_batch_sync(sg_batch *b, int *failed);
-/* Pass tiles of the batch's launches (one choice for all members), set or
- * tuned on the members' current states as sg_autotune does for a handle. */
+/* The same for a batch's launches, timed on the members' current states. */
 int sg_batch_set_tiles(sg_batch *b, const int narrow[3]);
 int sg_batch_get_tiles(sg_batch *b, int narrow[3]);
 int sg_batch_autotune(sg_batch *b, int reps, double *ms);

@@ -326,6 +326,14 @@ static int setup_params(sg_handle *h) {
   P.m4[0] = acoef4 / 4.0; P.m4[1] = bcoef4 / 4.0 / 4.0; P.m4[2] = ccoef4 / 4.0 / 9.0;
   P.m5[0] = acoef5 / 4.0; P.m5[1] = bcoef5 / 4.0 / 4.0; P.m5[2] = ccoef5 / 4.0 / 9.0;
   P.m5[3] = dcoef5 / 4.0 / 1.6e1;
+  for (int k = 0; k < 5; k++) {
+    P.id.ac[k] = P.ac[k]; P.id.sc[k] = P.sc[k]; P.id.mc[k] = P.mc[k];
+    P.is.ac[k] = (float)P.ac[k]; P.is.sc[k] = (float)P.sc[k]; P.is.mc[k] = (float)P.mc[k];
+  }
+  for (int d = 0; d < 3; d++) {
+    P.id.ovdel[d] = P.ovdel[d]; P.id.ovdl2[d] = P.ovdl2[d];
+    P.is.ovdel[d] = (float)P.ovdel[d]; P.is.ovdl2[d] = (float)P.ovdl2[d];
+  }
   P.thrd = 1.0 / 3.0; P.tthd = 2.0 * P.thrd; P.fthd = 2.0 * P.tthd;   // src/com_senga2.h:271-272
   // boundaries: y, z periodic; x periodic or NSBCI3 (left) + NSBCO1 (right)
   for (int f = 2; f < 6; f++)
@@ -395,7 +403,7 @@ static int mech_compiled(const sg_config &c, const Tables &t) {
   return memcmp(&t.nuw, &T::nuw, sizeof T::nuw) == 0;
 }
 
-static int init_launch(sg_handle *h, const int nw[3]) {
+static int init_launch(sg_handle *h) {
   if (h->lbase) {
     hipStreamSynchronize(h->stream);
     hipFree(h->lbase);
@@ -403,8 +411,7 @@ static int init_launch(sg_handle *h, const int nw[3]) {
   }
   Launch &L = h->L;
   memset(&L, 0, sizeof L);
-  for (int d = 0; d < 3; d++) L.pass_nw[d] = nw[d] ? 1 : 0;
-  member_blocks(h->P, L.pass_nw, L.nblk);
+  member_blocks(h->P, L.nblk);
   size_t bytes = (sizeof(Member) + 255) / 256 * 256;
   for (int k = 0; k < L_NKIND; k++) bytes += ((size_t)L.nblk[k] * sizeof(uint32_t) + 255) / 256 * 256;
   if (hipMalloc(&h->lbase, bytes) != hipSuccess) {
@@ -519,7 +526,7 @@ static int batch_prepare(sg_batch *b) {
   std::vector<std::array<int, L_NKIND>> nb(nm);
   for (int m = 0; m < nm; m++) {
     hm[m] = b->members[m]->mem;
-    member_blocks(b->members[m]->P, b->L.pass_nw, nb[m].data());
+    member_blocks(b->members[m]->P, nb[m].data());
     for (int k = 0; k < L_NKIND; k++) {
       hm[m].blk0[k] = tot[k];
       long t = (long)tot[k] + nb[m][k];
@@ -684,14 +691,11 @@ static size_t case_bytes(const Params &P, size_t *main_block) {
   const size_t tabsz = ((sizeof(Tables) + 255) / 256) * 256;
   const size_t main = bytes + itn + ((facesz + 255) / 256) * 256 + cfgsz + tabsz + 256;
   if (main_block) *main_block = main;
-  // block maps sized for the larger of the wide and narrow pass tiles
-  int nblk[L_NKIND], nb1[L_NKIND];
-  const int wide[3] = {0, 0, 0}, narrow[3] = {1, 1, 1};
-  member_blocks(P, wide, nblk);
-  member_blocks(P, narrow, nb1);
+  int nblk[L_NKIND];
+  member_blocks(P, nblk);
   size_t lb = (sizeof(Member) + 255) / 256 * 256;
   for (int k = 0; k < L_NKIND; k++)
-    lb += ((size_t)(nblk[k] > nb1[k] ? nblk[k] : nb1[k]) * sizeof(uint32_t) + 255) / 256 * 256;
+    lb += ((size_t)nblk[k] * sizeof(uint32_t) + 255) / 256 * 256;
   return main + lb;
 }
 
@@ -722,6 +726,7 @@ int sg_create(const sg_config *cfg, sg_handle **out) {
   if (rc) { delete h; return rc; }
   for (int r = 0; r < SG_NROW; r++) {
     row_weights(h->P, r, h->tab.roww[r]);
+    row_dense(h->tab.roww[r], r, h->tab.rowd[r]);
     mix_row_weights(h->P, r, h->tab.mixw[r]);
   }
   if (hipGetDevice(&h->device) != hipSuccess || hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking) != hipSuccess) {
@@ -776,8 +781,7 @@ int sg_create(const sg_config *cfg, sg_handle **out) {
   hipEventCreate(&h->ev[1]);
   h->scratch = noalloc_scratch(h->device);   // once per device; failure only disables the no-allocation call
   h->etime = 0.0;
-  const int wide[3] = {0, 0, 0};
-  if (init_launch(h, wide) != 0) {
+  if (init_launch(h) != 0) {
     sg_destroy(h);
     return SG_ENOMEM;
   }
@@ -910,7 +914,7 @@ static int eval_rhs(sg_handle *h) {
   if (!rc) rc = timed(h, K_PRIM, [&] { launch_prim(L, h->stream); });
   if (!rc) rc = timed(h, K_PASSX, [&] { launch_pass(0, L, h->stream); });
   if (!rc && L.radn) rc = timed(h, K_RADN, [&] { launch_radn(L, h->stream); });
-  if (!rc) rc = timed(h, K_PASSY, [&] { launch_pass(1, L, h->stream); });
+  if (!rc && L.nblk[L_PASSY]) rc = timed(h, K_PASSY, [&] { launch_pass(1, L, h->stream); });
   if (!rc) rc = timed(h, K_PASSZ, [&] { launch_pass(2, L, h->stream); });
   if (!rc && L.bndx) rc = timed(h, K_NSCBC, [&] { launch_nscbc(L, h->stream); });
   return rc;
@@ -1263,8 +1267,8 @@ int sg_batch_member(sg_batch *b, int idx, sg_handle **h) {
 
 }  // extern "C"
 
-// ---- Tile tuning ------------------------------------------------------------
-// A tuning run times launches on the live state.  It changes nothing a later
+// ---- Timing of the passes ---------------------------------------------------
+// A timing run launches the passes on the live state.  It changes nothing a later
 // step reads except the stored temperature (the Newton initial guess) and the
 // interval indices, which prim rewrites; those are saved and put back, so a
 // tuned run computes exactly what an untuned one does.
@@ -1322,8 +1326,8 @@ extern "C" {
 int sg_set_tiles(sg_handle *h, const int narrow[3]) {
   if (!h || !narrow) return SG_EINVAL;
   if (h->batch) return set_err(h, SG_ESTATE, "handle advances in a batch");
-  if (init_launch(h, narrow) != 0) return set_err(h, SG_ENOMEM, "launch table allocation failed");
-  return refresh_member(h);
+  for (int d = 0; d < 3; d++) h->L.pass_nw[d] = narrow[d] ? 1 : 0;
+  return 0;
 }
 
 int sg_mechanism_compiled(const sg_handle *h, int *compiled) {
@@ -1348,27 +1352,9 @@ int sg_autotune(sg_handle *h, int reps, double *ms) {
   if (rc) return rc;
   if (h->L.inflow) launch_boundt(h->L, h->stream);
   launch_prim(h->L, h->stream);
-  int nw[3] = {h->L.pass_nw[0], h->L.pass_nw[1], h->L.pass_nw[2]};
   double total = 0.0;
-  for (int d = 0; d < 3 && !rc; d++) {
-    double tb = 1e30;
-    int bw = nw[d];
-    for (int w = 0; w < 2 && !rc; w++) {
-      int cur[3] = {nw[0], nw[1], nw[2]};
-      cur[d] = w;
-      if (init_launch(h, cur) != 0) rc = set_err(h, SG_ENOMEM, "launch table allocation failed");
-      if (!rc) rc = refresh_member(h);
-      if (rc) break;
-      const double t = time_launches(h->stream, reps, [&] { launch_pass(d, h->L, h->stream); });
-      if (t < tb) { tb = t; bw = w; }
-    }
-    nw[d] = bw;
-    total += tb;
-  }
-  if (!rc && init_launch(h, nw) != 0) rc = set_err(h, SG_ENOMEM, "launch table allocation failed");
-  if (!rc) rc = refresh_member(h);
-  int rc2 = snap_restore(h, sn, h->stream);
-  if (!rc) rc = rc2;
+  for (int d = 0; d < 3; d++) total += time_launches(h->stream, reps, [&] { launch_pass(d, h->L, h->stream); });
+  rc = snap_restore(h, sn, h->stream);
   if (!rc) rc = refresh_member(h);
   if (!rc && ms) *ms = total;
   return rc;
@@ -1377,7 +1363,6 @@ int sg_autotune(sg_handle *h, int reps, double *ms) {
 int sg_batch_set_tiles(sg_batch *b, const int narrow[3]) {
   if (!b || !narrow) return SG_EINVAL;
   for (int d = 0; d < 3; d++) b->L.pass_nw[d] = narrow[d] ? 1 : 0;
-  b->dirty_layout = 1;
   return 0;
 }
 
@@ -1403,26 +1388,11 @@ int sg_batch_autotune(sg_batch *b, int reps, double *ms) {
     launch_prim(b->L, b->stream);
   }
   double total = 0.0;
-  for (int d = 0; d < 3 && !rc; d++) {
-    double tb = 1e30;
-    int bw = b->L.pass_nw[d];
-    for (int w = 0; w < 2 && !rc; w++) {
-      b->L.pass_nw[d] = w;
-      b->dirty_layout = 1;
-      rc = batch_prepare(b);
-      if (rc) break;
-      const double t = time_launches(b->stream, reps, [&] { launch_pass(d, b->L, b->stream); });
-      if (t < tb) { tb = t; bw = w; }
-    }
-    b->L.pass_nw[d] = bw;
-    total += tb;
-  }
-  b->dirty_layout = 1;
-  int rc2 = batch_prepare(b);
-  if (!rc) rc = rc2;
+  for (int d = 0; d < 3 && !rc; d++)
+    total += time_launches(b->stream, reps, [&] { launch_pass(d, b->L, b->stream); });
   for (size_t m = 0; m < b->members.size(); m++)
     if (sn[m].buf) {
-      rc2 = snap_restore(b->members[m], sn[m], b->stream);
+      int rc2 = snap_restore(b->members[m], sn[m], b->stream);
       if (!rc) rc = rc2;
     }
   if (!rc && ms) *ms = total;

@@ -10,6 +10,14 @@ namespace sg {
 
 constexpr int HALO = 5;
 
+// Interior stencil coefficients in a kernel's working precision: read as they
+// are from scalar registers (a uniform FP64 value converted in the kernel
+// lives in a vector register).
+template <class R>
+struct Interior {
+  R ac[5], sc[5], mc[5], ovdel[3], ovdl2[3];
+};
+
 // Grid, stencil coefficients and boundary flags handed to every kernel by
 // value.  Coefficients are the values src/dfinit.f:61-477 computes.
 struct Params {
@@ -22,6 +30,8 @@ struct Params {
   double ac[5], c1[4], c2[4], c3[2], c4[3], c5[4];       // first derivative
   double sc[5], s1[5], s2[5], s3[2], s4[3], s5[4];       // second derivative
   double mc[5], my1[2], m1[4], m2[4], m3[2], m4[3], m5[4];  // mixed
+  Interior<double> id;         // ac, sc, mc, ovdel, ovdl2 again, and in FP32
+  Interior<float> is;
   double thrd, tthd, fthd;
   // boundary flags per face xl,xr,yl,yr,zl,zr (src/bcinit.f)
   int fcnv[6], fvsn[6], fvst[6], fcon[6], fadb[6], fdif[6];
@@ -52,6 +62,7 @@ struct Params {
 #define SG_NROW 11    // derivative row kinds: interior, 5 left and 5 right closure rows
 struct Tables {
   double roww[SG_NROW][10];                      // 5-term row weights W1, W2 per row kind
+  double rowd[SG_NROW][20];                      // the same rows as weights of f(q) - f(0), q = -5..-1, 1..5: first, second
   double mixw[SG_NROW][7];                       // mixed-derivative row weights W0..W4, V0, V1
   double cp[SG_MAX_SPEC][SG_NTINT][SG_NCPMAX];   // amascp polynomial part
   double ct[SG_MAX_SPEC][SG_NTINT][SG_NCPMAX];   // amasct
@@ -153,12 +164,16 @@ struct Launch {
   int ns, precision, bndx, inflow;
   int ext;          // a molecular-transport option on: the passes with those terms
   int radn;         // some member has radiation on: the radiation kernel after the x pass
-  int pass_nw[3];   // pass tile per direction: 0 wide (rows of 32), 1 narrow (rows of 16)
+  int pass_nw[3];   // sg_set_tiles' flags (kept for sg_get_tiles; the passes have one tile)
   int mechfix;      // the chemistry is the compiled mechanism (MechH2): unrolled step loop
 };
 
+// Whether the x and y derivatives are formed in one pass: without the
+// molecular-transport options.
+inline bool pass_xy(const Params &P) { return !(P.mixw || P.mixp || P.soret || P.dufour); }
+
 // member block counts of each kind (sg_kernels.hip)
-void member_blocks(const Params &P, const int nw[3], int nblk[L_NKIND]);
+void member_blocks(const Params &P, int nblk[L_NKIND]);
 
 // launchers (sg_kernels.hip)
 void launch_tempin(const Params &P, const sg_config *dcfg, const Fields &F, hipStream_t st);

@@ -4,13 +4,15 @@
 //   k_boundt   BOUNDT inflow values at x-left            (src/boundt.f:177-218)
 //   k_prim     TEMPER + transport + CHRATE + enthalpies   (src/temper.f, src/chrate.f,
 //                                                          src/rhscal.f:515-573,1292-1470,3854-3891)
-//   k_pass<d>  every derivative along direction d and the RHS terms that
-//              involve derivatives along d only           (src/rhscal.f, src/rhsvel.f)
+//   k_pass     every derivative along x and y, then along z (or one direction
+//              each) and the RHS terms separable in them  (src/rhscal.f, src/rhsvel.f)
 //   k_final    mixed derivatives, cross-direction viscous terms, NSCBC face
 //              corrections (src/bounds.f) and the RK register update
 //              (src/lincom.f, src/fincom.f)
 // Periodic directions use wrapped indices: no halo copies are stored.
 #include <math.h>
+
+#include <type_traits>
 
 #include "sg_internal.h"
 #include "sg_stencil.h"
@@ -1518,24 +1520,36 @@ __global__ void __launch_bounds__(BLK) __attribute__((amdgpu_waves_per_eu(4))) k
 #pragma clang fp contract(fast)
 
 // ---------------------------------------------------------------------------
-// Direction pass: all derivatives along DIR and the RHS terms separable in
-// DIR.  The block owns a tile of points; every field (or product of fields)
-// is staged once into LDS with a 5-deep halo along DIR, then each thread
-// evaluates its stencils from LDS at compile-time offsets.  Fields staged:
-// rho u_d (resident for the whole pass), e, T, lambda, u, v, w, p - p_ref,
-// mu, h_mix and per species Y, rho D, h; the products with rho u_d that the
-// split convective forms difference (e rho u_d, Y rho u_d and the momentum
-// fluxes rho u_d u_b) are formed inside the stencils from two tiles.
-// Bounded x direction: the x pass runs as two launches.  Edge tiles, PASS_EW
+// Derivative passes: all derivatives along one direction, or along x and y,
+// and the RHS terms separable in them.  x with y, then z (with the
+// molecular-transport options: x, y and z each, whose terms take the
+// registers).
+//
+// A block owns a tile of 16 x 16 points; one of its waves takes the
+// hydrodynamic fields and every other one up to SPMAX species, each lane four
+// points in a row.  A wave stages its own fields one after the other into an
+// LDS tile of its own with a 5-deep halo and evaluates their stencils from
+// there, so the waves of a block run without barriers but for the resident
+// rho u_d tiles at the start and the sums over species at the end.  What
+// bounds this: one point per lane read 667 LDS values per point and direction
+// (59% of the LDS cycles of the y pass, 16 waves a CU), and a joint x-y pass
+// of that form held every species' sums of both directions in each lane and
+// spilled.  Four points per lane share a 14-value window along the rows (14
+// LDS reads instead of 40), and three species a wave leave the registers for
+// both directions.  At 128^3 (9 species) the passes took 0.335 (x) + 0.285
+// (y) + 0.295 (z) ms in FP64 and 0.217 + 0.157 + 0.166 ms in FP32; x with y
+// now takes 0.44 and z 0.265 ms in FP64, 0.27 and 0.15 in FP32, the x-y pass
+// reading the primitives once (1305 -> 790 B per point of HBM traffic).
+// Products with rho u_d (e rho u_d, Y rho u_d and the momentum fluxes rho u_d
+// u_b) are formed inside the stencils from two tiles.
+//
+// Bounded x direction: x passes run as two launches.  Edge tiles, PASS_EW
 // points wide at each end of a row, hold every closure row (i < 5, i > nx - 6)
-// and evaluate all their stencils in the uniform row form; interior tiles
+// and evaluate their x stencils with per-column weights; interior tiles
 // cover [PASS_EW, nx - PASS_EW), where every stencil is the interior one and
-// reaches no further than 5 points into the edge tiles.  Neither kernel then
-// carries the other's stencil code (with both in one kernel, and the form
-// chosen per wave, the bounded x pass took 0.345 ms at 128^3 in FP64; the
-// interior form alone 0.298 ms, the row form alone 0.331 ms).  xp: 0 every
-// x tile of a row (periodic x, and the y and z passes); 1 the interior tiles
-// of a bounded row; 2 its edge tiles.  Rows shorter than 2 PASS_EW are all edge
+// reaches no further than 5 points into the edge tiles.  xp: 0 every x tile
+// of a row (periodic x, and the y and z passes); 1 the interior tiles of a
+// bounded row; 2 its edge tiles.  Rows shorter than 2 PASS_EW are all edge
 // tiles.
 constexpr int PASS_EW = 16;
 __host__ __device__ inline int pass_xtiles(int nx, int xp, int tx) {
@@ -1550,554 +1564,783 @@ __host__ __device__ inline int pass_x0(int nx, int xp, int tx, int bx) {
   return nx >= 2 * PASS_EW ? (bx == 0 ? 0 : nx - PASS_EW) : bx * PASS_EW;
 }
 
-template <int DIR, int NW = 0, int XP = 0>
+// The block of a pass: a tile of 16 x-points times 16 rows along y (or along
+// z, DV = 2), worked by one wave for the hydrodynamic fields and one wave per
+// SPW species.  DX: the x derivatives; DV: the y (1) or z (2) derivatives.  A
+// pass takes x with y, or one direction.
+template <int DX, int DV, int NS, class R, bool EXT>
 struct PassTile {
-  // Wide tiles (NW = 0), x: 32x8 points (halo 42/32 along x); y, z: 32x16
-  // points, 512 threads, so that the 10-point halo along the pass direction
-  // costs 26/16 re-reads.  Narrow tiles (NW = 1) have rows of 16 points and
-  // twice the rows: no idle lanes when nx is an odd multiple of 16, and a
-  // cheaper y/z halo (42/32), at half-length coalesced rows.  The autotuner
-  // picks one per direction.  Edge tiles of a bounded x row (XP = 2):
-  // PASS_EW x 16 points.
-  static constexpr int TX = XP == 2 ? PASS_EW : (NW ? 16 : 32);
-  static constexpr int TY = XP == 2 ? 16 : (DIR == 0 ? (NW ? 16 : 8) : (DIR == 1 ? (NW ? 32 : 16) : 1));
-  static constexpr int TZ = DIR == 2 ? (NW ? 32 : 16) : 1;
-  static constexpr int NT = TX * TY * TZ;   // threads per block
-  static constexpr int LX = TX + (DIR == 0 ? 10 : 0);
-  static constexpr int LY = TY + (DIR == 1 ? 10 : 0);
-  static constexpr int LZ = TZ + (DIR == 2 ? 10 : 0);
-  static constexpr int LN = LX * LY * LZ;
-  static constexpr int LSTR = DIR == 0 ? 1 : (DIR == 1 ? LX : LX * LY);   // LDS stride along DIR
+  static constexpr int ND = DX + (DV != 0);
+  static constexpr int T = 16, NP = T * T;                 // points of the tile
+  static constexpr int HX = DX ? 5 : 0, HV = DV ? 5 : 0;   // halo
+  // species a wave: what its registers hold (a direction more costs another
+  // value per species and point)
+  static constexpr int SPMAX = ND == 2 ? 3 : 4;
+  static constexpr int NG = (NS + SPMAX - 1) / SPMAX;      // species waves
+  static constexpr int SPW = (NS + NG - 1) / NG;
+  static constexpr int NW = 1 + NG, NT = 64 * NW;
+  // LDS tile: rows padded so that the four rows a wave reads at once (4 apart)
+  // start on different banks
+  static constexpr int LXU = T + 2 * HX, LV = T + 2 * HV;
+  static constexpr int LX = DX ? (sizeof(R) == 8 ? 28 : 36) : 20;
+  static constexpr int LR = LX * LV;
+  static constexpr int LN = LXU * T + 2 * HV * T;          // staged values: no corners
+  static constexpr int NIT = (LN + 63) / 64;               // per lane of the staging wave
+  static constexpr int LS = LR + NIT * 64 - LN;            // the pad takes the surplus lanes' stores
+  static constexpr int NRED = 2 + ND;                      // sums over the waves: energy, vt, ucor per direction
+  // tile coordinates of staged value l: the rows with their x halo, then the
+  // rows of the halo along the other direction
+  static __device__ __forceinline__ void coords(int l, int &tx, int &tv) {
+    if (l < LXU * T) {
+      tx = l % LXU;
+      tv = HV + l / LXU;
+    } else {
+      const int m = l - LXU * T, r = m / T;
+      tx = HX + m % T;
+      tv = r < 5 ? r : r + T;
+    }
+  }
+  static __device__ __forceinline__ int slot(int l) {
+    if (l >= LN) return LR + l - LN;
+    int tx, tv;
+    coords(l, tx, tv);
+    return tv * LX + tx;
+  }
 };
 
-// Occupancy: FP64 passes need their 128 registers (4 waves per SIMD; at 5
-// the spills made the y and z passes 40% slower).  The FP32 passes are held
-// to 80 registers for 6 waves per SIMD (3 blocks per CU), which the
-// latency-bound staging pipeline turns into 7-10% shorter y and z passes and
-// 2% shorter interior x passes; the bounded-row edge tiles, which would spill
-// heavily at 80, keep 4, and so do the passes with the molar-mass and
-// pressure diffusion terms (EXT), which need more.
-template <int DIR, bool BND, int NS, class R, int NW, int XP = 0, bool EXT = false>
-__global__ void __launch_bounds__((PassTile<DIR, NW, XP>::NT))
-__attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 && XP != 2 && !EXT ? 6 : 4))) k_pass(const Member *__restrict__ mem,
-                                                                                                       const uint32_t *__restrict__ map) {
-  static_assert(XP == 0 || (DIR == 0 && (XP == 1) != BND), "interior x tiles take the periodic form, edge tiles the bounded one");
-  using T_ = PassTile<DIR, NW, XP>;
-  constexpr int TX = T_::TX, TY = T_::TY, LX = T_::LX, LY = T_::LY, LN = T_::LN, LSTR = T_::LSTR;
-  constexpr int NTH = T_::NT;
-  // LN staged values per field, padded to whole block-sized rows so that
-  // every thread loads and stores unconditionally
-  constexpr int NIT = (LN + NTH - 1) / NTH;
-  // Two buffers of up to STW fields each: a stage stages one field, or up to
-  // three fields under one barrier (e, T and lambda; u, v and w; p and mu; a
-  // species' Y_k, rho D_k and h_k).  Grouped stages were measured faster in
-  // every direction than one field per barrier (FP64 x pass at 128^3
-  // periodic: 0.279 -> 0.265 ms), a few FP64 spills included.
-  constexpr int STW = 3;
-  __shared__ R tile[2][STW][NIT * NTH];
-  const int t = threadIdx.x;
-  const int lx = t % TX, ly = (t / TX) % TY, lz = t / (TX * TY);
+// Registers: an FP64 wave holds its species' right-hand sides and gradients
+// of four points per lane (36 values with two directions) beside a 14-value
+// stencil window, which takes the 256 registers of two waves per SIMD (254 in
+// the x-y pass, 214-228 in z); FP32 fits three (x with y) and four waves.
+// With one spill per lane and field the z pass was 40% slower, hence the sums
+// kept in LDS and the branches that end in a barrier of their own.
+template <int DX, int DV, bool BND, int NS, class R, int XP = 0, bool EXT = false>
+__global__ void __launch_bounds__((PassTile<DX, DV, NS, R, EXT>::NT))
+__attribute__((amdgpu_waves_per_eu(sizeof(R) == 8 ? 2 : (DX + (DV != 0) == 2 ? 3 : 4)))) k_pass(
+    const Member *__restrict__ mem, const uint32_t *__restrict__ map) {
+  static_assert(XP == 0 || (DX && (XP == 1) != BND), "interior x tiles take the periodic form, edge tiles the bounded one");
+  static_assert(!EXT || DX + (DV != 0) == 1, "the passes with the transport options take one direction each");
+  using T_ = PassTile<DX, DV, NS, R, EXT>;
+  constexpr int ND = T_::ND, T = T_::T, HX = T_::HX, HV = T_::HV, LX = T_::LX, LN = T_::LN, NIT = T_::NIT,
+                NP = T_::NP, NW = T_::NW, NT = T_::NT, SPW = T_::SPW;
+  constexpr int KIND = XP == 2 ? L_PASSXE : (DX ? L_PASSX : (DV == 1 ? L_PASSY : L_PASSZ));
+  constexpr bool RMW = !DX;   // the x part writes the accumulators, the others add to them
+  const int t = threadIdx.x, lane = t & 63, wv = __builtin_amdgcn_readfirstlane(t >> 6);
   int lb;
-  const Member &M = member_at<XP == 2 ? L_PASSXE : L_PASSX + DIR>(mem, map, xcd_block(blockIdx.x, gridDim.x), lb);
+  const Member &M = member_at<KIND>(mem, map, xcd_block(blockIdx.x, gridDim.x), lb);
   const Params P = M.P;
   const Fields F = global_fields(M.F);
-  const int nbx = pass_xtiles(P.nx, XP, TX), nby = (P.ny + TY - 1) / TY;
-  const int x0 = pass_x0(P.nx, XP, TX, lb % nbx), y0 = ((lb / nbx) % nby) * TY, z0 = (lb / (nbx * nby)) * T_::TZ;
-  const int i = x0 + lx, j = y0 + ly, k = z0 + lz;
-  const bool active = i < (XP == 1 ? P.nx - PASS_EW : P.nx) && j < P.ny && k < P.nz;
-  const long idx = ((long)k * P.ny + j) * P.nx + i;
-  const int m = DIR == 0 ? i : (DIR == 1 ? j : k);
-  const int n = DIR == 0 ? P.nx : (DIR == 1 ? P.ny : P.nz);
-  // closure row of this point (bounded direction only)
-  Sten S;
-  S.mode = 0;
-  if (BND) {
-    if (m < 5) S.mode = 1 + m;
-    else if (m > n - 6 && m < n) S.mode = 11 + (n - 1 - m);
+  // tile origin: x0, and row v0 along y (z for DV = 2) in plane w0
+  const int nv = DV == 2 ? P.nz : P.ny, nw = DV == 2 ? P.ny : P.nz;
+  const int nbx = pass_xtiles(P.nx, XP, T), nbv = (nv + T - 1) / T;
+  int bv, w0;
+  if (DV == 2) {   // planes before rows of tiles, so that x rows of one z follow each other
+    w0 = (lb / nbx) % nw;
+    bv = lb / (nbx * nw);
+  } else {
+    bv = (lb / nbx) % nbv;
+    w0 = lb / (nbx * nbv);
   }
-  // Bounded direction: edge tiles (XP = 2) evaluate every stencil in the
-  // uniform 5-term row form (weights from an LDS table, offsets packed per
-  // lane; interior points there take the interior row, the same sums).
-  __shared__ R wtab[BND ? SG_NROW : 1][10];   // in the working precision
-  int pk[5] = {0, 0, 0, 0, 0};
-  int row = 0;
-  if (BND) {
-    if (t < SG_NROW * 10) (&wtab[0][0])[t] = (R)(&F.tab->roww[0][0])[t];
-    row = row_of_mode(S.mode);
-#pragma unroll
-    for (int q = 0; q < 5; q++) pk[q] = c_row_offsets.w[row][q];
-  }
-  // Row offsets for one stencil.  In FP64 each stencil takes fresh copies, so
-  // that its neighbour addresses are formed per stencil rather than held live
-  // for the whole pass (they made the FP64 x pass spill); the FP32 pass has
-  // the registers and is faster keeping them.
-  auto pkc = [&](int (&pq)[5]) {
-#pragma unroll
-    for (int q = 0; q < 5; q++) {
-      pq[q] = pk[q];
-      if constexpr (sizeof(R) == 8) asm volatile("" : "+v"(pq[q]));
-    }
+  const int x0 = pass_x0(P.nx, XP, T, lb % nbx), v0 = bv * T;
+  // this lane's points: column x, rows 4 q .. 4 q + 3 of the tile
+  const int lx = lane & 15, q4 = (lane >> 4) * 4;
+  const int i = x0 + lx;
+  const bool inx = i < (XP == 1 ? P.nx - PASS_EW : P.nx);
+  auto elem = [&](int x, int v) {
+    return (uint32_t)(((DV == 2 ? v : w0) * P.ny + (DV == 2 ? w0 : v)) * P.nx + x);
   };
-  // LDS position of this point
-  const int lbase = (lz + (DIR == 2 ? 5 : 0)) * LX * LY + (ly + (DIR == 1 ? 5 : 0)) * LX + lx + (DIR == 0 ? 5 : 0);
-  // staging: global source index of LDS slot l (wrap when periodic, clamp when bounded)
-  auto gsrc = [&](int l) -> long {
-    int tx = l % LX, ty = (l / LX) % LY, tz = l / (LX * LY);
-    int gx = x0 + tx - (DIR == 0 ? 5 : 0);
-    int gy = y0 + ty - (DIR == 1 ? 5 : 0);
-    int gz = z0 + tz - (DIR == 2 ? 5 : 0);
-    int g = DIR == 0 ? gx : (DIR == 1 ? gy : gz);
-    if (BND) {
-      g = g < 0 ? 0 : (g >= n ? n - 1 : g);
-    } else {
-      g = g < 0 ? g + n : (g >= n ? g - n : g);
-    }
-    if (DIR == 0) gx = g; else if (DIR == 1) gy = g; else gz = g;
-    gx = gx < P.nx ? gx : P.nx - 1;
-    gy = gy < P.ny ? gy : P.ny - 1;
-    gz = gz < P.nz ? gz : P.nz - 1;
-    return ((long)gz * P.ny + gy) * P.nx + gx;
+  auto active = [&](int r) { return inx && v0 + q4 + r < nv; };
+  // byte offset of point r in a field (past the end of a partial tile, of the
+  // last point inside: loads need no test, only stores do)
+  const int vend = nv - 1 - (v0 + q4);
+  const uint32_t pbs = (uint32_t)(DV == 2 ? P.ny * P.nx : P.nx) * (uint32_t)sizeof(R);
+  const uint32_t pb0 = elem(i < P.nx ? i : P.nx - 1, v0 + q4) * (uint32_t)sizeof(R);
+  auto pb = [&](int r) { return pb0 + (uint32_t)(r < vend ? r : vend) * pbs; };
+  // source element of staged value l (wrapped when periodic, clamped when
+  // bounded; a second clamp keeps what partial tiles do not use inside)
+  auto gsrc = [&](int l) {
+    int tx, tv;
+    T_::coords(l, tx, tv);
+    int gx = x0 + tx - HX, gv = v0 + tv - HV;
+    auto wrap = [](int g, int n) { return g < 0 ? g + n : (g >= n ? g - n : g); };
+    if (DX) gx = BND ? (gx < 0 ? 0 : gx) : wrap(gx, P.nx);
+    if (DV) gv = wrap(gv, nv);
+    return elem(gx < P.nx ? gx : P.nx - 1, gv < nv ? gv : nv - 1);
   };
-  int buf = 0;
-  // Stage one field (or product) into the current buffer.  One barrier per
-  // stage: the two buffers alternate, and the barrier of stage s orders the
-  // reads of stage s-1 before the writes of stage s+1 into the same buffer.
-  // Software pipeline: prefetch(fn) issues the global loads of the next
-  // field into registers; stage() stores them into the current buffer and
-  // synchronises.  Each stage's loads are thus in flight while the previous
-  // stage's stencils are evaluated.
-  R pf[STW][NIT];
-  auto prefetch_to = [&](int f, auto fn) {
-#pragma unroll
-    for (int it = 0; it < NIT; it++) {
-      const int l = t + it * NTH;
-      pf[f][it] = (R)fn(gsrc(l < LN ? l : LN - 1));
-    }
-  };
-  auto prefetch = [&](auto fn) { prefetch_to(0, fn); };
-  auto stage_n = [&](int nf) {
-#pragma unroll
-    for (int f = 0; f < STW; f++)
-      if (f < nf) {
-#pragma unroll
-        for (int it = 0; it < NIT; it++) tile[buf][f][t + it * NTH] = pf[f][it];
-      }
-    __syncthreads();
-  };
-  auto stage = [&]() { stage_n(1); };
-  auto wq = [&](int q) { return wtab[BND ? row : 0][q]; };
-  auto D1f = [&](int f) {
-    auto at = [&](int kk) { return tile[buf][f][lbase + (kk - 8) * LSTR]; };
-    auto fq = [&](int q) { return tile[buf][f][lbase + q * LSTR]; };
-    if (BND) { int pq[5]; pkc(pq); return d1_rows<R>(P, pq, DIR, wq, fq); }
-    return d1<false, R>(P, S, DIR, at);
-  };
-  auto D2f = [&](int f) {
-    auto at = [&](int kk) { return tile[buf][f][lbase + (kk - 8) * LSTR]; };
-    auto fq = [&](int q) { return tile[buf][f][lbase + q * LSTR]; };
-    if (BND) { int pq[5]; pkc(pq); return d2_rows<R>(P, pq, DIR, wq, fq); }
-    return d2<false, R>(P, S, DIR, at);
-  };
-  auto ctrf = [&](int f) { return tile[buf][f][lbase]; };
-  auto D1 = [&]() { return D1f(0); };
-  auto ctr = [&]() { return ctrf(0); };
-  auto next = [&]() { buf ^= 1; };
+  // rho u_d of the pass directions, 1/(mixture molar mass) (EXT), and what
+  // every wave needs per point: the divergence of rho u over the directions,
+  // and (EXT) the derivatives of ln W, ln p and ln T
+  __shared__ R tmd[ND][T_::LR];
+  __shared__ R tow[EXT ? T_::LR : 1];
+  __shared__ R tdiv[NP];
+  __shared__ R text[EXT ? 6 : 1][NP];
+  // one field per wave at a time
+  __shared__ R tbuf[NW][T_::LS];
+  R *const tb = tbuf[wv];
+  // the waves' sums at every point: energy, divergence of the correction
+  // velocity and its components.  Each lane keeps its own points' sums here
+  // (24 to 32 registers fewer), and the waves' are added at the end.
+  __shared__ R tsum[NW][T_::NRED][NP];
   const long fs = P.fstride;
-  const double *Q = F.q;
   const R *pr = (const R *)F.prim;
-  const double *mx = Q + fs, *my = Q + 2 * fs, *mz = Q + 3 * fs;
-  const double *md = DIR == 0 ? mx : (DIR == 1 ? my : mz);
-  const R *uu = pr + P_U * fs, *vv = pr + P_V * fs, *ww = pr + P_W * fs;
-  const R *ee = pr + P_E * fs, *TT = pr + P_T * fs, *pp = pr + P_P * fs;
-  const R *la = pr + P_LAM * fs, *mu = pr + P_MU * fs, *hm = pr + P_HMIX * fs;
-  const R pref = pp[0];   // PRUN(IPREF,JPREF,KPREF), src/rhsvel.f:741
-  // boundary-plane flags of this direction (src/bcinit.f)
-  const bool atL = BND && m == 0, atR = BND && m == n - 1;
-  const int fl = 2 * DIR, fr = 2 * DIR + 1;
-  auto zf = [&](const int *flag) { return (atL && flag[fl]) || (atR && flag[fr]); };
-  const bool zcon = zf(P.fcon), zdif = zf(P.fdif), zadb = zf(P.fadb), zvsn = zf(P.fvsn),
-             zvst = zf(P.fvst);
-  const bool zdifadb = zdif || zadb;
-  // ADB zeroing of the correction-velocity divergence acts on any face plane
-  const bool zadb_any = (i == 0 && P.fadb[0]) || (i == P.nx - 1 && P.fadb[1]) ||
-                        (j == 0 && P.fadb[2]) || (j == P.ny - 1 && P.fadb[3]) ||
-                        (k == 0 && P.fadb[4]) || (k == P.nz - 1 && P.fadb[5]);
+  // a wave's own staging: fetch() issues the loads of a field into registers,
+  // put() stores them to the wave's tile.  No barrier: LDS accesses of a wave
+  // take effect in order, and no other wave touches the tile.  The next
+  // field's loads are in flight while this one's stencils are evaluated.
+  uint32_t go[NIT];
+#pragma unroll
+  for (int it = 0; it < NIT; it++) {
+    const int l = lane + 64 * it;
+    go[it] = gsrc(l < LN ? l : LN - 1) * (uint32_t)sizeof(R);
+  }
+  uint32_t slots[(NIT + 1) / 2];   // LDS positions, two to a register
+#pragma unroll
+  for (int it = 0; it < NIT; it += 2)
+    slots[it / 2] = (uint32_t)T_::slot(lane + 64 * it) | (it + 1 < NIT ? (uint32_t)T_::slot(lane + 64 * (it + 1)) << 16 : 0u);
+  // fields in flight: two where the registers allow it (FP64 z pass 277 ->
+  // 267 us at 128^3; FP32 spilled, 154 -> 164 us)
+  constexpr int DEPTH = !EXT && !DX && sizeof(R) == 8 ? 2 : 1;
+  R pf[DEPTH][NIT];
+  auto fetch = [&](int k, const R *src) {
+#pragma unroll
+    for (int it = 0; it < NIT; it++) pf[k % DEPTH][it] = fld(src, go[it]);
+  };
+  auto put_v = [&](const R (&val)[NIT]) {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int it = 0; it < NIT; it++) tb[(slots[it / 2] >> (16 * (it & 1))) & 0xffff] = val[it];
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  };
+  auto put = [&](int k) { put_v(pf[k % DEPTH]); };
+  // the k-th field of a wave: of the hydrodynamic wave, and (without the
+  // transport options, whose stages depend on the species) of a species wave
+  const int s0 = (wv - 1) * SPW;   // first species of a species wave
+  auto has = [&](int q) { return NS % SPW == 0 || s0 + q < NS; };
+  auto fetch_h = [&](int k) {
+    constexpr int order[9] = {P_MU, P_P, P_LAM, P_T, P_E, P_U, P_V, P_W, P_HMIX};
+    if (k < 9) fetch(k, pr + order[k] * fs);
+  };
+  auto fetch_s = [&](int k) {
+    const int sp = s0 + k / 3;
+    if (k < 3 * SPW && has(k / 3))
+      fetch(k, pr + (k % 3 == 0 ? prim_rd(P, sp) : (k % 3 == 1 ? prim_y(P, sp) : prim_h(P, sp))));
+  };
+  // bounded x: the tile columns' closure rows, as weights of f(q) - f(0),
+  // q = -5..-1, 1..5 (first and second derivative)
+  __shared__ R wrow[BND ? 20 : 1][T];
+  if (BND) {
+    for (int e = t; e < 20 * T; e += NT) {
+      const int x = x0 + e % T;
+      const int row = x < 5 ? 1 + x : (x > P.nx - 6 && x < P.nx ? 6 + (P.nx - 1 - x) : 0);
+      wrow[e / T][e % T] = (R)F.tab->rowd[row][e / T];
+    }
+  }
+  // rho u_d (and 1/W) to LDS by all waves together; their loads go out first,
+  // then those of each wave's first fields
+  constexpr int NMD = (LN + NT - 1) / NT;
+  R mreg[ND + EXT][NMD];
+#pragma unroll
+  for (int it = 0; it < NMD; it++) {
+    const int l = t + it * NT;
+    const uint32_t g = gsrc(l < LN ? l : LN - 1);
+#pragma unroll
+    for (int dd = 0; dd < ND; dd++)
+      mreg[dd][it] = (R)fld(F.q + (long)(1 + (DX && dd == 0 ? 0 : DV)) * fs, g * 8u);
+    if constexpr (EXT) mreg[ND][it] = fld(pr + (long)P_OVW * fs, g * (uint32_t)sizeof(R));
+  }
+#pragma unroll
+  for (int k = 0; k < DEPTH; k++) {
+    if (wv == 0) fetch_h(k);
+    else fetch_s(k);
+  }
+#pragma unroll
+  for (int it = 0; it < NMD; it++) {
+    const int l = t + it * NT;
+    if (l < LN) {
+      const int s = T_::slot(l);
+#pragma unroll
+      for (int dd = 0; dd < ND; dd++) tmd[dd][s] = mreg[dd][it];
+      if constexpr (EXT) tow[s] = mreg[ND][it];
+    }
+  }
+  const Interior<R> &C = interior(P, R(0));
+  // LDS position of the first row of this lane's window (5 rows before its
+  // first point when the pass has a row direction), and of its point r
+  const int lw = q4 * LX + lx + HX;
+  auto lp = [&](int r) { return lw + (r + HV) * LX; };
+  constexpr int VD = ND - 1;   // index of the row direction
+  // First and second derivative, and first derivative of the product with
+  // rho u_d, of a staged field at the lane's four points: along the rows from
+  // one window of 14 values, along x from a window of 11 per point.
+  // WANT: bit 0 first, bit 1 second derivative, bit 2 derivative of the
+  // product; each (direction, point) is handed to use(dd, r, g1, g2, gp) as it
+  // is formed, so that no set of results is held
+  auto ders = [&](auto want, const R *tile, R (&c)[4], auto use) {
+    constexpr int W = decltype(want)::value;
+    if constexpr (DV != 0) {
+      R wn[14];
+#pragma unroll
+      for (int k = 0; k < 14; k++) wn[k] = tile[lw + k * LX];
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        c[r] = wn[r + 5];
+        pin(c[r]);
+      }
+      R a1[4], a2[4];
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        auto at = [&](int kk) { return wn[r + kk - 3]; };
+        a1[r] = W & 1 ? d1_in<R>(C, DV, at) : R(0);
+        a2[r] = W & 2 ? d2_in<R>(C, DV, at) : R(0);
+        if (W & 4) {
+          if (W & 1) pin(a1[r]);
+          if (W & 2) pin(a2[r]);
+        } else {
+          use(VD, r, a1[r], a2[r], R(0));
+        }
+      }
+      if (W & 4) {
+#pragma unroll
+        for (int k = 0; k < 14; k++) wn[k] = wn[k] * tmd[VD][lw + k * LX];
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+          use(VD, r, a1[r], a2[r], d1_in<R>(C, DV, [&](int kk) { return wn[r + kk - 3]; }));
+      }
+      SG_PHASE();
+    } else {
+#pragma unroll
+      for (int r = 0; r < 4; r++) c[r] = tile[lp(r)];
+    }
+    if constexpr (DX != 0 && BND) {
+      // closure rows: the column's weights one after the other, over the four
+      // points; the next neighbour's values are read while this one's are used
+      R s1[4], s2[4], sp[4], cm[4], v[2][4];
+      auto read = [&](int q) {
+        const int e = q & 1, o = q < 5 ? q - 5 : q - 4;
+#pragma unroll
+        for (int r = 0; r < 4; r++) v[e][r] = tile[lp(r) + o];
+      };
+      read(0);
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        s1[r] = s2[r] = sp[r] = R(0);
+        cm[r] = W & 4 ? c[r] * tmd[0][lp(r)] : R(0);
+      }
+#pragma unroll
+      for (int q = 0; q < 10; q++) {
+        const int e = q & 1, o = q < 5 ? q - 5 : q - 4;
+        R m[4];
+        if (W & 4) {
+#pragma unroll
+          for (int r = 0; r < 4; r++) m[r] = tmd[0][lp(r) + o];
+        }
+        const R wa = wrow[q][lx], wb = W & 2 ? wrow[10 + q][lx] : R(0);
+        if (q < 9) read(q + 1);
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+          const R f = v[e][r] - c[r];
+          if (W & 1) s1[r] = s1[r] + wa * f;
+          if (W & 2) s2[r] = s2[r] + wb * f;
+          if (W & 4) sp[r] = sp[r] + wa * (v[e][r] * m[r] - cm[r]);
+        }
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+          if (W & 1) pin(s1[r]);
+          if (W & 2) pin(s2[r]);
+          if (W & 4) pin(sp[r]);
+        }
+        SG_PHASE();
+      }
+#pragma unroll
+      for (int r = 0; r < 4; r++) use(0, r, s1[r] * C.ovdel[0], s2[r] * C.ovdl2[0], sp[r] * C.ovdel[0]);
+    } else if constexpr (DX != 0) {
+      // interior rows: the five pairs of neighbours one after the other, over
+      // the four points (a window per point would hold more values); the next
+      // pair's values are read while this one's are used
+      R s1[4], s2[4], sp[4], fp[2][4], fm[2][4];
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        fp[0][r] = tile[lp(r) + 1];
+        fm[0][r] = tile[lp(r) - 1];
+      }
+#pragma unroll
+      for (int q = 0; q < 5; q++) {
+        const int e = q & 1;
+        R gp[4], gm[4];
+        if (W & 4) {
+#pragma unroll
+          for (int r = 0; r < 4; r++) {
+            gp[r] = tmd[0][lp(r) + q + 1];
+            gm[r] = tmd[0][lp(r) - q - 1];
+          }
+        }
+        if (q < 4) {
+#pragma unroll
+          for (int r = 0; r < 4; r++) {
+            fp[e ^ 1][r] = tile[lp(r) + q + 2];
+            fm[e ^ 1][r] = tile[lp(r) - q - 2];
+          }
+        }
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+          const R p = fp[e][r], m = fm[e][r];
+          if (W & 1) s1[r] = q ? s1[r] + C.ac[q] * (p - m) : C.ac[q] * (p - m);
+          if (W & 2) {
+            const R f = (p - c[r]) - (c[r] - m);
+            s2[r] = q ? s2[r] + C.sc[q] * f : C.sc[q] * f;
+          }
+          if (W & 4) {
+            const R f = p * gp[r] - m * gm[r];
+            sp[r] = q ? sp[r] + C.ac[q] * f : C.ac[q] * f;
+          }
+        }
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+          if (W & 1) pin(s1[r]);
+          if (W & 2) pin(s2[r]);
+          if (W & 4) pin(sp[r]);
+        }
+        SG_PHASE();
+      }
+#pragma unroll
+      for (int r = 0; r < 4; r++)
+        use(0, r, W & 1 ? s1[r] * C.ovdel[0] : R(0), W & 2 ? s2[r] * C.ovdl2[0] : R(0),
+            W & 4 ? sp[r] * C.ovdel[0] : R(0));
+    }
+  };
+  using W1 = std::integral_constant<int, 1>;
+  using W12 = std::integral_constant<int, 3>;
+  using W14 = std::integral_constant<int, 5>;
+  using W124 = std::integral_constant<int, 7>;
+  auto dir = [](int dd) { return DX && dd == 0 ? 0 : DV; };
+  // boundary-plane flags of the x direction (src/bcinit.f; y and z are
+  // periodic), false in every other direction
+  const bool atL = BND && i == 0, atR = BND && i == P.nx - 1;
+  auto zf = [&](const int *flag, int dd) { return BND && dd == 0 && ((atL && flag[0]) || (atR && flag[1])); };
+  // ADB zeroing of the correction-velocity divergence acts on the face planes
+  const bool zadb_any = (i == 0 && P.fadb[0]) || (i == P.nx - 1 && P.fadb[1]);
   // x-face point of an NSCBC case: copies of what the NSCBC kernel reads go
-  // to the face arrays (in the x pass only the edge tiles hold such points;
-  // the test and the address are formed where they are used, so that they
-  // hold no registers through the pass)
-  constexpr bool FACES = DIR != 0 || XP == 2;
-  auto facew = [&]() { return FACES && active && (P.inflow_xl || P.outflow_xr) && (i == 0 || i == P.nx - 1); };
+  // to the face arrays (of the tiles of a bounded x direction only the edge
+  // tiles hold such points)
+  constexpr bool FACES = !DX || XP == 2;
+  auto facew = [&](int r) {
+    return FACES && active(r) && (P.inflow_xl || P.outflow_xr) && (i == 0 || i == P.nx - 1);
+  };
   const long fnf = (long)P.ny * P.nz;
-  auto fcw = [&](int slot) -> double & {
+  auto fcw = [&](int slot, int r) -> double & {
+    const int v = v0 + q4 + r, j = DV == 2 ? w0 : v, k = DV == 2 ? v : w0;
     return F.face[(i == 0 ? 0 : (long)nface(P.ns) * fnf) + (long)slot * fnf + (long)k * P.ny + j];
   };
-  // rho u_d stays resident in its own LDS tile for the whole pass: products
-  // with it (e rho u_d, Y rho u_d and the momentum fluxes rho u_d u_b) are
-  // formed inside the stencils from two staged tiles instead of being staged
-  // from memory, which is the same multiplication of the same two values.
-  __shared__ R tmd[NIT * NTH];
-  // EXT: 1/(mixture molar mass), resident for the species' pressure diffusion
-  __shared__ R tow[EXT ? NIT * NTH : 1];
-  auto stage_md = [&]() {
-#pragma unroll
-    for (int it = 0; it < NIT; it++) {
-      tmd[t + it * NTH] = pf[0][it];
-      if constexpr (EXT) tow[t + it * NTH] = pf[1][it];
-    }
-    __syncthreads();
-  };
-  auto atm = [&](int kk) { return tmd[lbase + (kk - 8) * LSTR]; };
-  auto fqm = [&](int q) { return tmd[lbase + q * LSTR]; };
-  auto D1M = [&]() {
-    if (BND) { int pq[5]; pkc(pq); return d1_rows<R>(P, pq, DIR, wq, fqm); }
-    return d1<false, R>(P, S, DIR, atm);
-  };
-  // The product stencil reads twice the operands of a plain one; its loads
-  // are kept from being hoisted over the preceding stencils so that they do
-  // not hold registers alongside them.
-  auto D1Pf = [&](int f) {
-    auto atp = [&](int kk) {
-      const int l = lbase + (kk - 8) * LSTR;
-      return tile[buf][f][l] * tmd[l];
-    };
-    auto fqp = [&](int q) {
-      const int l = lbase + q * LSTR;
-      return tile[buf][f][l] * tmd[l];
-    };
-    SG_PHASE();
-    R r;
-    if (BND) { int pq[5]; pkc(pq); r = d1_rows<R>(P, pq, DIR, wq, fqp); }
-    else r = d1<false, R>(P, S, DIR, atp);
-    pin(r);
-    SG_PHASE();
-    return r;
-  };
-  // EXT: rho D_k Y_k (pw: times 1 - W_k / W) differentiated along this
-  // direction, from the staged Y_k (slot 0) and rho D_k (slot 1) tiles and
-  // the resident 1/W tile, formed at every stencil point as the reference
-  // forms STORE7 (src/rhscal.f:1977, 2374)
-  auto D1PY = [&](bool pw, R wk) {
-    auto val = [&](int l) {
-      R v = tile[buf][1][l] * tile[buf][0][l];
-      if (pw) v = v * (R(1) - wk * tow[l]);
-      return v;
-    };
-    auto atp = [&](int kk) { return val(lbase + (kk - 8) * LSTR); };
-    auto fqp = [&](int q) { return val(lbase + q * LSTR); };
-    SG_PHASE();
-    R r;
-    if (BND) { int pq[5]; pkc(pq); r = d1_rows<R>(P, pq, DIR, wq, fqp); }
-    else r = d1<false, R>(P, S, DIR, atp);
-    pin(r);
-    SG_PHASE();
-    return r;
-  };
-  // Momentum fluxes rho u_d u_b of the pass direction d: all three are formed
-  // inside the stencils from the resident rho u_d tile and the staged u_b
-  // tile.  The reference forms the fluxes rho u*v (in y), rho u*w and rho v*w
-  // (in z) as rho u_b * u_d (src/rhsvel.f:348-729); rho u_d * u_b is the same
-  // quantity, rounded differently in its last bit, and needs no staged
-  // product (one barrier and two field loads fewer in y, two and four in z).
-  R flux[3];
-  R dm, md0, aD, aE, dp, p0, dmu, mu0;
-  R du[3], d2u[3], u0[3];
-  auto prefetch_species = [&](int sp) {
-    const R *Ys = pr + prim_y(P, sp), *Rs = pr + prim_rd(P, sp), *Hs = pr + prim_h(P, sp);
-    prefetch_to(0, [Ys](long g) { return Ys[g]; });
-    prefetch_to(1, [Rs](long g) { return Rs[g]; });
-    prefetch_to(2, [Hs](long g) { return Hs[g]; });
-  };
-  auto f_pp = [&](long g) { return pp[g] - pref; };
-  auto f_mu = [&](long g) { return mu[g]; };
-  const R *lw = pr + P_LNW * fs, *lp = pr + P_LNP * fs, *ow = pr + P_OVW * fs, *lt = pr + P_LNT * fs;
-  prefetch([&](long g) { return md[g]; });
-  if constexpr (EXT) prefetch_to(1, [&](long g) { return ow[g]; });
-  stage_md();
-  // e, T and lambda under one barrier, u, v and w under the next, then
-  // p - p_ref and mu
-  prefetch_to(0, [&](long g) { return ee[g]; });
-  prefetch_to(1, [&](long g) { return TT[g]; });
-  prefetch_to(2, [&](long g) { return la[g]; });
-  dm = D1M(); md0 = tmd[lbase];
-  pin(dm); pin(md0);
-  aD = -dm;
-  stage_n(3);
-  prefetch_to(0, [&](long g) { return uu[g]; });
-  prefetch_to(1, [&](long g) { return vv[g]; });
-  prefetch_to(2, [&](long g) { return ww[g]; });
-  // ---------------- continuity and energy convection (src/rhscal.f:141-415)
-  {
-    R dem = D1Pf(0);
-    const R de = D1f(0);
-    const R e0 = ctrf(0);
-    aE = -R(0.5) * (e0 * dm + dem + md0 * de);
-    pin(aE);
-    if (DIR == 0 && facew()) {
-      fcw(F_E) = (double)e0;
-      fcw(F_T) = (double)ctrf(1);
-      fcw(F_P) = (double)pp[idx];
-      fcw(F_RHO) = Q[idx];
-    }
-  }
-  SG_PHASE();
-  // ---------------- heat conduction (src/rhscal.f:427-797)
-  {
-    R dT = D1f(1), d2T = D2f(1);
-    pin(dT); pin(d2T);
-    SG_PHASE();
-    const R dl = D1f(2);
-    const R lam0 = ctrf(2);
-    aE = aE + (zcon ? R(0) : dl) * dT;
-    aE = aE + lam0 * (zcon ? R(0) : d2T);
-    pin(aE);
-  }
-  next();
-  // ---------------- velocity derivatives and rho u_d u_b fluxes, all three
-  // from the resident rho u_d tile and the staged u_b tiles
-  stage_n(3);
-  prefetch_to(0, f_pp);
-  prefetch_to(1, f_mu);
-#pragma unroll
-  for (int a = 0; a < 3; a++) {
-    du[a] = D1f(a); d2u[a] = D2f(a); u0[a] = ctrf(a);
-    pin(du[a]); pin(d2u[a]); pin(u0[a]);
-    flux[a] = D1Pf(a);
-    pin(flux[a]);
-    SG_PHASE();
-  }
-  if (facew()) {
-    if (DIR == 0) {
-#pragma unroll
-      for (int a = 0; a < 3; a++) {
-        fcw(F_U + a) = (double)u0[a];
-        fcw(F_DUX + a) = (double)du[a];
+  __syncthreads();
+  // the divergence of rho u, each row of the lanes' points by one wave
+  for (int r = wv; r < 4; r += NW) {
+    R dm = R(0);
+    if constexpr (DX != 0) {
+      const R *m = tmd[0] + lp(r);
+      if constexpr (BND) {
+        for (int q = 0; q < 10; q++) dm = dm + wrow[q][lx] * (m[q < 5 ? q - 5 : q - 4] - m[0]);
+        dm = dm * C.ovdel[0];
+      } else {
+        dm = d1_in<R>(C, 0, [&](int kk) { return m[kk - 8]; });
       }
-    } else if (DIR == 1) {
-      fcw(F_DUY) = (double)du[0];
-      fcw(F_DVY) = (double)du[1];
-    } else {
-      fcw(F_DUZ) = (double)du[0];
-      fcw(F_DWZ) = (double)du[2];
+    }
+    if constexpr (DV != 0) {
+      const R d = d1_in<R>(C, DV, [&](int kk) { return tmd[VD][lp(r) + (kk - 8) * LX]; });
+      dm = DX ? dm + d : d;
+    }
+    tdiv[(q4 + r) * T + lx] = dm;
+  }
+  // EXT: first and second derivatives of ln W, ln p and ln(T/TDIFGB)
+  // (src/rhscal.f:945-1004), the three fields spread over the species waves
+  if constexpr (EXT) {
+    if (wv > 0) {
+      R hold[NIT];
+#pragma unroll
+      for (int it = 0; it < NIT; it++) hold[it] = pf[0][it];
+      for (int f = wv - 1; f < 3; f += NW - 1) {
+        fetch(0, pr + (f == 0 ? P_LNW : (f == 1 ? P_LNP : P_LNT)) * fs);
+        put(0);
+        R c[4];
+        ders(W12{}, tb, c, [&](int, int r, R g1, R g2, R) {
+          text[2 * f][(q4 + r) * T + lx] = g1;
+          text[2 * f + 1][(q4 + r) * T + lx] = g2;
+        });
+      }
+#pragma unroll
+      for (int it = 0; it < NIT; it++) pf[0][it] = hold[it];
     }
   }
-  next();
-  // ---------------- p - p_ref and mu under one barrier
-  stage_n(2);
-  if constexpr (EXT) {
-    prefetch_to(0, [&](long g) { return lw[g]; });
-    prefetch_to(1, [&](long g) { return lp[g]; });
-    prefetch_to(2, [&](long g) { return lt[g]; });
-  } else {
-    prefetch_species(0);
+  __syncthreads();
+  auto divm = [&](int r) { return tdiv[(q4 + r) * T + lx]; };
+  auto md0 = [&](int dd, int r) { return tmd[dd][lp(r)]; };
+  R *A = (R *)F.acc;
+  R *const ts = &tsum[wv][0][q4 * T + lx];
+  auto sum_at = [&](int v, int r) -> R & { return ts[v * NP + r * T]; };
+  R aE[4];
+#pragma unroll
+  for (int r = 0; r < 4; r++) {
+    aE[r] = R(0);
+    if (wv > 0) {
+#pragma unroll
+      for (int v = 1; v < T_::NRED; v++) sum_at(v, r) = R(0);
+    }
   }
-  dp = D1f(0); p0 = ctrf(0);
-  dmu = D1f(1); mu0 = ctrf(1);
-  next();
-  pin(dmu); pin(mu0);
-  // ---------------- EXT: ln W, ln p and ln(T/TDIFGB) under one barrier
-  // (src/rhscal.f:945-1004); 1/W went into its resident tile with rho u_d
-  R dlw = R(0), d2lw = R(0), dlp = R(0), d2lp = R(0), dlt = R(0), d2lt = R(0);
-  if constexpr (EXT) {
-    stage_n(3);
-    prefetch_species(0);
-    dlw = D1f(0); d2lw = D2f(0);
-    dlp = D1f(1); d2lp = D2f(1);
-    dlt = D1f(2); d2lt = D2f(2);
-    pin(dlw); pin(d2lw); pin(dlp); pin(d2lp); pin(dlt); pin(d2lt);
-    next();
-  }
-  // ---------------- momentum convection (src/rhsvel.f:348-729, 1312-2110)
-  R aM[3];
-  {
-    const R r0 = active ? (R)Q[idx] : R(0);
+  // The waves' sums, added over the species waves: divergence of the
+  // correction velocity and its components.  Every wave passes exactly one
+  // barrier here, each on its own side of the branch below, so that neither
+  // side's values hold registers on the other.
+  R vt[4], uc[ND][4];
+  auto add_waves = [&]() {
+#pragma unroll
+    for (int r = 0; r < 4; r++) sum_at(0, r) = aE[r];
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      const int p = (q4 + r) * T + lx;
+      vt[r] = R(0);
+#pragma unroll
+      for (int dd = 0; dd < ND; dd++) uc[dd][r] = R(0);
+#pragma unroll
+      for (int w = 1; w < NW; w++) {
+        vt[r] = vt[r] + tsum[w][1][p];
+#pragma unroll
+        for (int dd = 0; dd < ND; dd++) uc[dd][r] = uc[dd][r] + tsum[w][2 + dd][p];
+      }
+    }
+  };
+  if (wv == 0) {
+    R hm0[4], ghm[ND][4];
+    // accumulator v of the hydrodynamic wave's point r; what a pass adds to is
+    // loaded before the stencils, so that no store waits for it
+    R oldh[RMW ? 5 : 1][4];
+    if (RMW) {
+#pragma unroll
+      for (int v = 0; v < 5; v++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) oldh[RMW ? v : 0][r] = fld(A + (long)v * fs, pb(r));
+    }
+    auto add = [&](int v, int r, R x) { fld(A + (long)v * fs, pb(r)) = RMW ? oldh[RMW ? v : 0][r] + x : x; };
+    // ---------------- hydrodynamic fields: mu, p, lambda, T, e, u, v, w, h_mix
+    R c[4], mu0[4], p0[4], dp[ND][4];
+    put(0);
+    fetch_h(DEPTH);
+    ders(W1{}, tb, mu0, [&](int dd, int r, R g1, R, R) {
+      if (active(r)) fld((R *)F.grad + (long)dir(dd) * fs, pb(r)) = g1;   // for the final kernel
+    });
+    // pressure, less PRUN(IPREF,JPREF,KPREF) (src/rhsvel.f:741)
+    const R pref = pr[(long)P_P * fs];
+#pragma unroll
+    for (int it = 0; it < NIT; it++) pf[1 % DEPTH][it] = pf[1 % DEPTH][it] - pref;
+    put(1);
+    fetch_h(1 + DEPTH);
+    ders(W1{}, tb, p0, [&](int dd, int r, R g1, R, R) {
+      dp[dd][r] = g1;
+      pin(dp[dd][r]);
+      if (facew(r)) fcw(dir(dd) == 0 ? F_DPDX : (dir(dd) == 1 ? F_DPDY : F_DPDZ), r) = (double)g1;
+    });
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      if (DX && facew(r)) {
+        fcw(F_P, r) = (double)fld(pr + (long)P_P * fs, pb(r));
+        fcw(F_RHO, r) = fld(F.q, pb(r) * (uint32_t)(8 / sizeof(R)));
+      }
+      p0[r] = p0[r] + pref + (R)P.pofs;   // stored pressure is p - pofs
+    }
+    // heat conduction (src/rhscal.f:427-797)
+    put(2);
+    fetch_h(2 + DEPTH);
+    {
+      R lam[4], dl[ND][4];
+      ders(W1{}, tb, lam, [&](int dd, int r, R g1, R, R) {
+        dl[dd][r] = zf(P.fcon, dd) ? R(0) : g1;
+        pin(dl[dd][r]);
+      });
+      put(3);
+      fetch_h(3 + DEPTH);
+      ders(W12{}, tb, c, [&](int dd, int r, R g1, R g2, R) {
+        aE[r] = aE[r] + dl[dd][r] * g1 + lam[r] * (zf(P.fcon, dd) ? R(0) : g2);
+        pin(aE[r]);
+      });
+      if (DX) {
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+          if (facew(r)) fcw(F_T, r) = (double)c[r];
+      }
+    }
+    // continuity and energy convection (src/rhscal.f:141-415)
+    put(4);
+    fetch_h(4 + DEPTH);
+    ders(W14{}, tb, c, [&](int dd, int r, R g1, R, R gp) {
+      aE[r] = aE[r] - R(0.5) * (gp + md0(dd, r) * g1);
+      pin(aE[r]);
+    });
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      aE[r] = aE[r] - R(0.5) * c[r] * divm(r);
+      pin(aE[r]);
+      if (DX && facew(r)) fcw(F_E, r) = (double)c[r];
+      if (active(r)) add(0, r, -divm(r));
+    }
+    // momentum: split convection from the resident rho u_d tiles and the
+    // staged u_b (src/rhsvel.f:348-729, 1312-2110; the reference forms the
+    // fluxes rho u*v in y, rho u*w and rho v*w in z as rho u_b * u_d: the
+    // same quantity, rounded differently in its last bit), pressure gradient
+    // and work (src/rhsvel.f:741-917), separable viscous terms
+    // (src/rhsvel.f:1462-2305)
 #pragma unroll
     for (int a = 0; a < 3; a++) {
-      if (a == DIR) aM[a] = -R(0.5) * (md0 * du[a] + flux[a] + u0[a] * dm);
-      else aM[a] = -R(0.5) * (flux[a] + u0[a] * dm) - R(0.5) * r0 * u0[DIR] * du[a];
-      pin(aM[a]);
-    }
-  }
-  // ---------------- pressure gradient and pressure work (src/rhsvel.f:741-917)
-  {
-    p0 = p0 + pref + (R)P.pofs;   // stored pressure is p - pofs
-    aM[DIR] = aM[DIR] - dp;
-    aE = aE - u0[DIR] * dp - p0 * du[DIR];
-    pin(aM[DIR]); pin(aE);
-    if (facew()) fcw(DIR == 0 ? F_DPDX : (DIR == 1 ? F_DPDY : F_DPDZ)) = dp;
-  }
-  // ---------------- separable viscous terms (src/rhsvel.f:1462-2305)
+      R s[4], tv[4];
 #pragma unroll
-  for (int a = 0; a < 3; a++) {
-    R tv;
-    if (a == DIR) tv = zvsn ? R(0) : mu0 * (R)P.fthd * d2u[a];
-    else tv = zvst ? R(0) : mu0 * d2u[a];
-    aM[a] = aM[a] + tv;
-    aE = aE + tv * u0[a];
-    pin(aM[a]);
-  }
-  pin(aE);
-  if (active) ((R *)F.grad)[(long)DIR * fs + idx] = dmu;   // d mu / d x_DIR for the final kernel
-  // ---------------- species (src/rhscal.f:1030-3944)
-  R vt = 0.0, ucor = 0.0;
-  R aY[NS], dYz[NS], yv[NS];
-#pragma unroll
-  for (int sp = 0; sp < NS; sp++) {
-    R dY, d2Y, yc, dYm, drD, rdc, dh, hc;
-    stage_n(3);
-    // a light species under Soret or Dufour stages TDRMIX and T * TDRMIX next
-    const bool ltsp = EXT && ((P.ltmask >> sp) & 1u);
-    auto prefetch_next = [&]() {
-      if (sp + 1 < NS) prefetch_species(sp + 1);
-      else prefetch([&](long g) { return hm[g]; });
-    };
-    if (ltsp) {
-      const R *Ts = pr + prim_tdr(P, sp), *TTs = pr + prim_tt(P, sp);
-      prefetch_to(0, [Ts](long g) { return Ts[g]; });
-      prefetch_to(1, [TTs](long g) { return TTs[g]; });
-    } else {
-      prefetch_next();
-    }
-    dY = D1f(0); d2Y = D2f(0); yc = ctrf(0);
-    pin(dY); pin(d2Y); pin(yc);
-    dYm = D1Pf(0);
-    pin(dYm);
-    SG_PHASE();
-    drD = D1f(1); rdc = ctrf(1);
-    pin(drD); pin(rdc);
-    SG_PHASE();
-    dh = D1f(2);
-    hc = ctrf(2);
-    R ds7w = R(0), ds7p = R(0), fw = R(0);
-    if constexpr (EXT) {
-      if (P.mixw) ds7w = D1PY(false, R(0));
-      if (P.mixp) {
-        const R wk = (R)F.tab->wmol[sp];
-        fw = R(1) - wk * tow[lbase];
-        ds7p = D1PY(true, wk);
-      }
-    }
-    next();
-    // EXT, light species: TDRMIX (slot 0) and T * TDRMIX (slot 1) of this
-    // species under one more barrier, the Y_k and rho D_k tiles still in the
-    // other buffer
-    R tdr0 = R(0), ds7s = R(0), dtt = R(0), ttc = R(0);
-    if constexpr (EXT) {
-      if (ltsp) {
-        stage_n(2);
-        prefetch_next();
-        const int pb = buf ^ 1;
-        tdr0 = ctrf(0);
-        ttc = ctrf(1);
-        if (P.dufour) dtt = D1f(1);
-        if (P.soret) {
-          // d(rho D_k Y_k TDRMIX)/dx_d as the reference forms STORE7 (src/rhscal.f:2768)
-          auto val = [&](int l) { return tile[pb][1][l] * tile[pb][0][l] * tile[buf][0][l]; };
-          auto atp = [&](int kk) { return val(lbase + (kk - 8) * LSTR); };
-          auto fqp = [&](int q) { return val(lbase + q * LSTR); };
-          SG_PHASE();
-          if (BND) { int pq[5]; pkc(pq); ds7s = d1_rows<R>(P, pq, DIR, wq, fqp); }
-          else ds7s = d1<false, R>(P, S, DIR, atp);
-          SG_PHASE();
-          // this stencil read the other buffer, which the next stage
-          // overwrites: every wave's reads end before any wave's stores
-          // (the barrier of this stage ordered only the stage before)
-          __syncthreads();
+      for (int r = 0; r < 4; r++) s[r] = tv[r] = R(0);
+      put(5 + a);
+      fetch_h(5 + a + DEPTH);
+      ders(W124{}, tb, c, [&](int dd, int r, R g1, R g2, R gp) {
+        const int d = dir(dd);
+        s[r] = s[r] - R(0.5) * (gp + md0(dd, r) * g1);
+        const R f = a == d ? mu0[r] * (R)P.fthd : mu0[r];
+        tv[r] = tv[r] + (zf(a == d ? P.fvsn : P.fvst, dd) ? R(0) : f * g2);
+        if (a == d) {
+          s[r] = s[r] - dp[dd][r];
+          aE[r] = aE[r] - c[r] * dp[dd][r] - p0[r] * g1;
+          pin(aE[r]);
         }
-        pin(tdr0); pin(ttc); pin(dtt); pin(ds7s);
-        next();
+        pin(s[r]); pin(tv[r]);
+        if (facew(r)) {
+          if (d == 0) fcw(F_DUX + a, r) = (double)g1;
+          if (d == 1 && a < 2) fcw(F_DUY + a, r) = (double)g1;
+          if (d == 2 && a != 1) fcw(a == 0 ? F_DUZ : F_DWZ, r) = (double)g1;
+        }
+      });
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        aE[r] = aE[r] + tv[r] * c[r];
+        pin(aE[r]);
+        if (active(r)) add(1 + a, r, s[r] + tv[r] - R(0.5) * c[r] * divm(r));
+        if (DX && facew(r)) fcw(F_U + a, r) = (double)c[r];
       }
     }
-    // Dufour: the species enthalpy carries R_k T TDRMIX through the heat-flux
-    // terms up to the Soret terms (src/rhscal.f:1549-1566, 2832-2845)
-    const bool dfsp = EXT && ltsp && P.dufour;
-    const R rgk = dfsp ? (R)F.tab->rgs[sp] : R(0);
-    const R hcu = dfsp ? hc + rgk * ttc : hc;
-    const R dhu = dfsp ? dh + rgk * dtt : dh;
-    R ys = -R(0.5) * yc * dm - R(0.5) * dYm - R(0.5) * md0 * dY;
-    const R g1 = (zdif ? R(0) : drD) * dY;
-    const R g2 = rdc * (zdif ? R(0) : d2Y);
-    ys = ys + g1 + g2;
-    vt = vt + g1 + g2;
-    aE = aE + hcu * ((zdifadb ? R(0) : drD) * dY);
-    aE = aE + ((zdifadb ? R(0) : dhu) * dY) * rdc;
-    aE = aE + (rdc * (zdifadb ? R(0) : d2Y)) * hcu;
-    ucor = ucor + rdc * dY;
-    if constexpr (EXT) {
-      // molar-mass (src/rhscal.f:1970-2364) and pressure (2365-2759)
-      // diffusion terms of this direction.  The heat-flux term with the
-      // species enthalpy gradient takes rho D_k in its x component, where the
-      // reference's STORE4 holds it at that point instead of dh/dx
-      // (src/rhscal.f:1887, 2071-2103, 2467-2499).
-      const R s7w = rdc * yc;
-      auto term = [&](R s7, R ds7, R d1l, R d2l, R ut, R dut) {
-        ucor = ucor + s7 * d1l;
-        const R f1 = (zdif ? R(0) : ds7) * d1l;
-        ys = ys + f1;
-        vt = vt + f1;
-        aE = aE + ((zdifadb ? R(0) : ds7) * d1l) * ut;
-        aE = aE + ((zdifadb ? R(0) : dut) * d1l) * s7;
-        const R f3 = (zdif ? R(0) : d2l) * s7;
-        ys = ys + f3;
-        vt = vt + f3;
-        aE = aE + ((zdifadb ? R(0) : d2l) * s7) * ut;
-      };
-      const R dhx = DIR == 0 ? rdc : dhu;
-      if (P.mixw) term(s7w, ds7w, dlw, d2lw, hcu, dhx);
-      if (P.mixp) term(s7w * fw, ds7p, dlp, d2lp, hcu, dhx);
-      // Soret (src/rhscal.f:2757-3758): rho D_k Y_k TDRMIX with ln(T/TDIFGB);
-      // its heat-flux terms take the species enthalpy without the Dufour part
-      // and its gradient afresh
-      if (ltsp && P.soret) term(s7w * tdr0, ds7s, dlt, d2lt, hc, dh);
-      pin(ys); pin(vt); pin(ucor); pin(aE);
-    }
-    aY[sp] = ys;
-    dYz[sp] = zdif ? R(0) : dY;
-    yv[sp] = yc;
-    pin(aY[sp]); pin(dYz[sp]); pin(yv[sp]); pin(vt); pin(ucor); pin(aE);
-    if (DIR == 0 && BND && facew()) {
-      fcw(F_NSCAL + sp) = dY;
-      fcw(face_h(P.ns, sp)) = (double)hc;
-      fcw(face_y(P.ns, sp)) = (double)yc;
-      fcw(face_rate(P.ns, sp)) = (double)((const R *)F.rate)[sp * fs + idx];
-    }
-  }
-  {
-    stage();
-    const R dhm = D1();
-    const R hm0 = ctr();
-    aE = aE - hm0 * (zadb_any ? R(0) : vt) - (zdifadb ? R(0) : dhm) * ucor;
-  }
-  if (!active) return;
-  // ---------------- store
-  // Every value the stores add to (the chemical rates in x, the accumulators
-  // in y and z) is loaded before the first store: the stores could alias
-  // those loads as far as the compiler knows, so a load after a store would
-  // cost a memory round trip per variable.
-  R *A = (R *)F.acc;
-  R ay[NS];
+    put(8);
+    ders(W1{}, tb, hm0, [&](int dd, int r, R g1, R, R) {
+      ghm[dd][r] = zf(P.fdif, dd) || zf(P.fadb, dd) ? R(0) : g1;
+      pin(ghm[dd][r]);
+    });
+    add_waves();
 #pragma unroll
-  for (int sp = 0; sp < NS; sp++) ay[sp] = aY[sp] - yv[sp] * vt - dYz[sp] * ucor;
-  R old[5 + NS];
-  if (DIR == 0) {
+    for (int r = 0; r < 4; r++) {
+      const int p = (q4 + r) * T + lx;
 #pragma unroll
-    for (int sp = 0; sp < NS; sp++) old[5 + sp] = ((const R *)F.rate)[sp * fs + idx];
-    A[idx] = aD;
-    A[fs + idx] = aM[0];
-    A[2 * fs + idx] = aM[1];
-    A[3 * fs + idx] = aM[2];
-    A[4 * fs + idx] = aE;
+      for (int w = 1; w < NW; w++) aE[r] = aE[r] + tsum[w][0][p];
+      aE[r] = aE[r] - hm0[r] * (zadb_any ? R(0) : vt[r]);
+#pragma unroll
+      for (int dd = 0; dd < ND; dd++) aE[r] = aE[r] - ghm[dd][r] * uc[dd][r];
+      if (active(r)) add(4, r, aE[r]);
+    }
   } else {
+    R aY[SPW][4], dYz[ND][SPW][4];
+    // ---------------- species (src/rhscal.f:1030-3944)
 #pragma unroll
-    for (int v = 0; v < 5 + NS; v++) old[v] = A[v * fs + idx];
-    A[idx] = old[0] + aD;
-    A[fs + idx] = old[1] + aM[0];
-    A[2 * fs + idx] = old[2] + aM[1];
-    A[3 * fs + idx] = old[3] + aM[2];
-    A[4 * fs + idx] = old[4] + aE;
+    for (int q = 0; q < SPW; q++) {
+      const int sp = s0 + q;
+      if (!has(q)) break;
+      R c[4], rd[4], drD[ND][4];
+      R er[EXT ? NIT : 1];
+      if constexpr (EXT) {
+#pragma unroll
+        for (int it = 0; it < NIT; it++) er[it] = pf[0][it];
+      }
+      put(3 * q);
+      if (EXT) fetch(0, pr + prim_y(P, sp));
+      else fetch_s(3 * q + DEPTH);
+      ders(W1{}, tb, rd, [&](int dd, int r, R g1, R, R) {
+        drD[dd][r] = g1;
+        pin(drD[dd][r]);
+      });
+      if constexpr (EXT) {
+#pragma unroll
+        for (int it = 0; it < NIT; it++) er[it] = er[it] * pf[0][it];   // rho D_k Y_k, staged below
+      }
+      put(3 * q + 1);
+      if (EXT) fetch(0, pr + prim_h(P, sp));
+      else fetch_s(3 * q + 1 + DEPTH);
+      // dif: the diffusive flux divergence without the correction velocity;
+      // dife: as it enters the energy
+      R dif[4], dife[4];
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        aY[q][r] = dif[r] = dife[r] = R(0);
+      }
+      ders(W124{}, tb, c, [&](int dd, int r, R g1, R g2, R gp) {
+        aY[q][r] = aY[q][r] - R(0.5) * (gp + md0(dd, r) * g1);
+        const R g = drD[dd][r] * g1 + rd[r] * g2;
+        dif[r] = dif[r] + (zf(P.fdif, dd) ? R(0) : g);
+        if (BND) dife[r] = dife[r] + (zf(P.fdif, dd) || zf(P.fadb, dd) ? R(0) : g);
+        sum_at(2 + dd, r) += rd[r] * g1;
+        dYz[dd][q][r] = g1;
+        pin(aY[q][r]); pin(dif[r]); pin(dYz[dd][q][r]);
+        if (BND) pin(dife[r]);
+        if (DX && dd == 0 && facew(r)) fcw(F_NSCAL + sp, r) = (double)g1;
+      });
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        aY[q][r] = aY[q][r] + dif[r] - R(0.5) * c[r] * divm(r);
+        sum_at(1, r) += dif[r];
+        if (!BND) dife[r] = dif[r];
+        pin(aY[q][r]);
+        if (DX && facew(r)) {
+          fcw(face_y(P.ns, sp), r) = (double)c[r];
+          fcw(face_rate(P.ns, sp), r) = (double)fld((const R *)F.rate + (long)sp * fs, pb(r));
+        }
+      }
+      put(3 * q + 2);
+      const bool more = q + 1 < SPW && has(q + 1);
+      const bool ltsp = EXT && ((P.ltmask >> sp) & 1u);
+      if (EXT) {
+        if (ltsp) fetch(0, pr + prim_tdr(P, sp));
+        else if (more) fetch(0, pr + prim_rd(P, sp + 1));
+      } else {
+        fetch_s(3 * q + 2 + DEPTH);
+      }
+      R h[4];
+      if constexpr (!EXT) {
+        ders(W1{}, tb, h, [&](int dd, int r, R g1, R, R) {
+          const bool z = zf(P.fdif, dd) || zf(P.fadb, dd);
+          aE[r] = aE[r] + ((z ? R(0) : g1) * dYz[dd][q][r]) * rd[r];
+          pin(aE[r]);
+        });
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+          aE[r] = aE[r] + h[r] * dife[r];
+          pin(aE[r]);
+          if (DX && facew(r)) fcw(face_h(P.ns, sp), r) = (double)h[r];
+#pragma unroll
+          for (int dd = 0; dd < ND; dd++) dYz[dd][q][r] = zf(P.fdif, dd) ? R(0) : dYz[dd][q][r];
+        }
+      } else {
+        R dh[4], dhu[4], hu[4], rdY[4], tdr[4], gt[4];
+        ders(W1{}, tb, h, [&](int, int r, R g1, R, R) {
+          dh[r] = g1;
+          pin(dh[r]);
+        });
+        const bool zdif = zf(P.fdif, 0), zdifadb = zdif || zf(P.fadb, 0);
+        // one transport option: flux s7 * grad(l), its derivative ds, with
+        // the enthalpy ut and its derivative dut
+        auto term = [&](int r, R s7, R ds, R d1l, R d2l, R ut, R dut) {
+          sum_at(2, r) += s7 * d1l;
+          const R f = ds * d1l + d2l * s7;
+          const R m = zdif ? R(0) : f, me = zdifadb ? R(0) : f;
+          aY[q][r] = aY[q][r] + m;
+          sum_at(1, r) += m;
+          aE[r] = aE[r] + me * ut + (zdifadb ? R(0) : dut) * d1l * s7;
+          pin(aY[q][r]); pin(aE[r]);
+        };
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+          if (DX && facew(r)) fcw(face_h(P.ns, sp), r) = (double)h[r];
+          hu[r] = h[r];
+          dhu[r] = dh[r];
+          rdY[r] = rd[r] * c[r];
+        }
+        if (ltsp) {
+          // TDRMIX and T * TDRMIX of this species.  Dufour: the species
+          // enthalpy carries R_k T TDRMIX through the heat-flux terms up to
+          // the Soret terms (src/rhscal.f:1549-1566, 2832-2845).  Soret:
+          // rho D_k Y_k TDRMIX with ln(T/TDIFGB) (src/rhscal.f:2757-3758),
+          // differentiated as the reference forms STORE7 (src/rhscal.f:2768);
+          // its heat-flux terms take the species enthalpy without the Dufour
+          // part
+          R e7[NIT];
+#pragma unroll
+          for (int it = 0; it < NIT; it++) e7[it] = er[it] * pf[0][it];
+          put(0);
+          fetch(0, pr + prim_tt(P, sp));
+#pragma unroll
+          for (int r = 0; r < 4; r++) {
+            tdr[r] = tb[lp(r)];
+            pin(tdr[r]);
+          }
+          R dum[4];
+          if (P.soret) {
+            put_v(e7);
+            ders(W1{}, tb, dum, [&](int, int r, R g1, R, R) {
+              gt[r] = g1;
+              pin(gt[r]);
+            });
+          }
+          put(0);
+          if (more) fetch(0, pr + prim_rd(P, sp + 1));
+          if (P.dufour) {
+            const R rgk = (R)F.tab->rgs[sp];
+            ders(W1{}, tb, dum, [&](int, int r, R g1, R, R) {
+              dhu[r] = dh[r] + rgk * g1;
+              pin(dhu[r]);
+            });
+#pragma unroll
+            for (int r = 0; r < 4; r++) hu[r] = h[r] + rgk * dum[r];
+          }
+        }
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+          aE[r] = aE[r] + hu[r] * dife[r] + (zdifadb ? R(0) : dhu[r]) * dYz[0][q][r] * rd[r];
+          dYz[0][q][r] = zdif ? R(0) : dYz[0][q][r];
+          pin(aE[r]); pin(dYz[0][q][r]);
+        }
+        auto ex = [&](int f, int r) { return text[f][(q4 + r) * T + lx]; };
+        // molar-mass (src/rhscal.f:1970-2364) and pressure (2365-2759)
+        // diffusion.  The heat-flux term with the species enthalpy gradient
+        // takes rho D_k in its x component, where the reference's STORE4
+        // holds it at that point instead of dh/dx (src/rhscal.f:1887,
+        // 2071-2103, 2467-2499).
+        R dum[4];
+        if (P.mixw) {
+          put_v(er);
+          ders(W1{}, tb, dum, [&](int, int r, R g1, R, R) {
+            term(r, rdY[r], g1, ex(0, r), ex(1, r), hu[r], DX ? rd[r] : dhu[r]);
+          });
+        }
+        if (P.mixp) {
+          const R wk = (R)F.tab->wmol[sp];
+#pragma unroll
+          for (int it = 0; it < NIT; it++) {
+            const int l = lane + 64 * it;
+            er[it] = er[it] * (R(1) - wk * tow[l < LN ? T_::slot(l) : 0]);
+          }
+          put_v(er);
+          ders(W1{}, tb, dum, [&](int, int r, R g1, R, R) {
+            term(r, rdY[r] * (R(1) - wk * tow[lp(r)]), g1, ex(2, r), ex(3, r), hu[r], DX ? rd[r] : dhu[r]);
+          });
+        }
+        if (ltsp && P.soret) {
+#pragma unroll
+          for (int r = 0; r < 4; r++) term(r, rdY[r] * tdr[r], gt[r], ex(4, r), ex(5, r), h[r], dh[r]);
+        }
+      }
+    }
+    // what the stores add to, and the points' own Y_k (read again instead of
+    // held through the pass), loaded before the barrier and the first store
+    R old[SPW][4], y0[SPW][4];
+#pragma unroll
+    for (int q = 0; q < SPW; q++)
+#pragma unroll
+      for (int r = 0; r < 4; r++)
+        if (has(q)) {
+          old[q][r] = fld((DX ? (const R *)F.rate : A + 5 * fs) + (long)(s0 + q) * fs, pb(r));
+          y0[q][r] = fld(pr + prim_y(P, s0 + q), pb(r));
+        }
+    add_waves();
+#pragma unroll
+    for (int q = 0; q < SPW; q++) {
+      if (!has(q)) break;
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        R s = aY[q][r] - y0[q][r] * vt[r];
+#pragma unroll
+        for (int dd = 0; dd < ND; dd++) s = s - dYz[dd][q][r] * uc[dd][r];
+        if (active(r)) fld(A + (long)(5 + s0 + q) * fs, pb(r)) = old[q][r] + s;
+      }
+    }
   }
-#pragma unroll
-  for (int sp = 0; sp < NS; sp++) A[(5 + sp) * fs + idx] = old[5 + sp] + ay[sp];
 }
 
 // ---------------------------------------------------------------------------
@@ -2641,37 +2884,32 @@ void launch_prim_t(const Launch &L, hipStream_t st) {
     else hipLaunchKernelGGL((k_tdr<NS, double>), g, b, 0, st, L.mem, L.map[L_POINT], L.c);
   }
 }
-template <int NS, class R, int NW, bool EXT>
-static void launch_pass_w(int dir, const Launch &L, hipStream_t st) {
-  const int k = L_PASSX + dir;
-  if (dir == 0) {
-    const dim3 b(PassTile<0, NW>::NT);
+template <int NS, class R, int DX, int DV, bool EXT>
+static void launch_pass_w(const Launch &L, hipStream_t st) {
+  const int k = DX ? L_PASSX : (DV == 1 ? L_PASSY : L_PASSZ);
+  const dim3 b(PassTile<DX, DV, NS, R, EXT>::NT);
+  if constexpr (DX != 0) {
     if (L.bndx) {
       // interior tiles of the bounded rows, then their edge tiles
       if (L.nblk[k] > 0)
-        hipLaunchKernelGGL((k_pass<0, false, NS, R, NW, 1, EXT>), dim3(L.nblk[k]), b, 0, st, L.mem, L.map[k]);
-      hipLaunchKernelGGL((k_pass<0, true, NS, R, 0, 2, EXT>), dim3(L.nblk[L_PASSXE]), dim3(PassTile<0, 0, 2>::NT), 0,
-                         st, L.mem, L.map[L_PASSXE]);
-    } else {
-      hipLaunchKernelGGL((k_pass<0, false, NS, R, NW, 0, EXT>), dim3(L.nblk[k]), b, 0, st, L.mem, L.map[k]);
+        hipLaunchKernelGGL((k_pass<DX, DV, false, NS, R, 1, EXT>), dim3(L.nblk[k]), b, 0, st, L.mem, L.map[k]);
+      hipLaunchKernelGGL((k_pass<DX, DV, true, NS, R, 2, EXT>), dim3(L.nblk[L_PASSXE]), b, 0, st, L.mem,
+                         L.map[L_PASSXE]);
+      return;
     }
-  } else if (dir == 1) {
-    hipLaunchKernelGGL((k_pass<1, false, NS, R, NW, 0, EXT>), dim3(L.nblk[k]), dim3(PassTile<1, NW>::NT), 0, st,
-                       L.mem, L.map[k]);
-  } else {
-    hipLaunchKernelGGL((k_pass<2, false, NS, R, NW, 0, EXT>), dim3(L.nblk[k]), dim3(PassTile<2, NW>::NT), 0, st,
-                       L.mem, L.map[k]);
   }
+  hipLaunchKernelGGL((k_pass<DX, DV, false, NS, R, 0, EXT>), dim3(L.nblk[k]), b, 0, st, L.mem, L.map[k]);
 }
-// EXT: the passes with the molar-mass and pressure diffusion terms
+// x with y and z, or (EXT, the passes with the molecular-transport options) x, y and z
 template <int NS, class R>
 static void launch_pass_r(int dir, const Launch &L, hipStream_t st) {
   if (L.ext) {
-    if (L.pass_nw[dir]) launch_pass_w<NS, R, 1, true>(dir, L, st);
-    else launch_pass_w<NS, R, 0, true>(dir, L, st);
+    if (dir == 0) launch_pass_w<NS, R, 1, 0, true>(L, st);
+    else if (dir == 1) launch_pass_w<NS, R, 0, 1, true>(L, st);
+    else launch_pass_w<NS, R, 0, 2, true>(L, st);
   } else {
-    if (L.pass_nw[dir]) launch_pass_w<NS, R, 1, false>(dir, L, st);
-    else launch_pass_w<NS, R, 0, false>(dir, L, st);
+    if (dir == 0) launch_pass_w<NS, R, 1, 1, false>(L, st);
+    else if (dir == 2) launch_pass_w<NS, R, 0, 2, false>(L, st);
   }
 }
 template <int NS>
@@ -2750,7 +2988,7 @@ __global__ void __launch_bounds__(BLK) k_zero(double *p, long n) {
   if (idx < n) p[idx] = 0.0;
 }
 
-void member_blocks(const Params &P, const int nw[3], int nblk[L_NKIND]) {
+void member_blocks(const Params &P, int nblk[L_NKIND]) {
   nblk[L_FACE] = (int)grid_for((long)P.ny * P.nz);
   nblk[L_FACE2] = (int)((2L * P.ny * P.nz + NSCBC_BLK - 1) / NSCBC_BLK);
   nblk[L_POINT] = (int)grid_for(P.npts);
@@ -2758,16 +2996,14 @@ void member_blocks(const Params &P, const int nw[3], int nblk[L_NKIND]) {
     return ((P.nx + tx - 1) / tx) * ((P.ny + ty - 1) / ty) * ((P.nz + tz - 1) / tz);
   };
   nblk[L_FINAL] = tiles(FinalTile::FX, FinalTile::FY, FinalTile::FZ);
-  // x pass: every tile of a row (periodic x), or the interior tiles of the
-  // bounded rows (L_PASSX) and their edge tiles (L_PASSXE)
-  const int xp = P.bnd[0] ? 1 : 0;
-  const int txw = nw[0] ? PassTile<0, 1>::TX : PassTile<0, 0>::TX, tyw = nw[0] ? PassTile<0, 1>::TY : PassTile<0, 0>::TY;
-  nblk[L_PASSX] = pass_xtiles(P.nx, xp, txw) * ((P.ny + tyw - 1) / tyw) * P.nz;
-  nblk[L_PASSXE] = P.bnd[0] ? pass_xtiles(P.nx, 2, PASS_EW) * ((P.ny + PassTile<0, 0, 2>::TY - 1) / PassTile<0, 0, 2>::TY) * P.nz : 0;
-  nblk[L_PASSY] = nw[1] ? tiles(PassTile<1, 1>::TX, PassTile<1, 1>::TY, PassTile<1, 1>::TZ)
-                        : tiles(PassTile<1, 0>::TX, PassTile<1, 0>::TY, PassTile<1, 0>::TZ);
-  nblk[L_PASSZ] = nw[2] ? tiles(PassTile<2, 1>::TX, PassTile<2, 1>::TY, PassTile<2, 1>::TZ)
-                        : tiles(PassTile<2, 0>::TX, PassTile<2, 0>::TY, PassTile<2, 0>::TZ);
+  // passes: every tile of a row (periodic x), or the interior tiles of the
+  // bounded rows (L_PASSX) and their edge tiles (L_PASSXE); y goes with x
+  // where the launch has no transport options
+  const long rows = (long)((P.ny + 15) / 16) * P.nz;
+  nblk[L_PASSX] = (int)(pass_xtiles(P.nx, P.bnd[0] ? 1 : 0, 16) * rows);
+  nblk[L_PASSXE] = P.bnd[0] ? (int)(pass_xtiles(P.nx, 2, 16) * rows) : 0;
+  nblk[L_PASSY] = pass_xy(P) ? 0 : tiles(16, 16, 1);
+  nblk[L_PASSZ] = tiles(16, 1, 16);
 }
 
 void launch_errmax(const Params &P, const Fields &F, hipStream_t st) {

@@ -140,6 +140,25 @@ __device__ __forceinline__ R d2(const Params &P, const Sten &S, int dir, Fn f) {
   return r * (R)P.ovdl2[dir];
 }
 
+// The interior rows of d1 and d2 with the coefficients in the working
+// precision (the same sums).
+__device__ __forceinline__ const Interior<double> &interior(const Params &P, double) { return P.id; }
+__device__ __forceinline__ const Interior<float> &interior(const Params &P, float) { return P.is; }
+
+template <class R, class Fn>
+__device__ __forceinline__ R d1_in(const Interior<R> &C, int dir, Fn f) {
+  const R fa = FQ(1) - FQ(-1), fb = FQ(2) - FQ(-2), fc = FQ(3) - FQ(-3), fd = FQ(4) - FQ(-4), fe = FQ(5) - FQ(-5);
+  return (C.ac[0] * fa + C.ac[1] * fb + C.ac[2] * fc + C.ac[3] * fd + C.ac[4] * fe) * C.ovdel[dir];
+}
+template <class R, class Fn>
+__device__ __forceinline__ R d2_in(const Interior<R> &C, int dir, Fn f) {
+  const R c = FQ(0);
+  const R ap = FQ(1) - c, am = c - FQ(-1), bp = FQ(2) - c, bm = c - FQ(-2), cp = FQ(3) - c, cm = c - FQ(-3),
+          dp = FQ(4) - c, dm = c - FQ(-4), ep = FQ(5) - c, em = c - FQ(-5);
+  return (C.sc[0] * (ap - am) + C.sc[1] * (bp - bm) + C.sc[2] * (cp - cm) + C.sc[3] * (dp - dm) +
+          C.sc[4] * (ep - em)) * C.ovdl2[dir];
+}
+
 #undef FQ
 
 // ---------------------------------------------------------------------------
@@ -198,6 +217,23 @@ inline void row_weights(const Params &P, int row, double *w) {
     case 3: case 8: for (int k = 0; k < 2; k++) { w[k] = P.c3[k]; w[5 + k] = P.s3[k]; } break;
     case 4: case 9: for (int k = 0; k < 3; k++) { w[k] = P.c4[k]; w[5 + k] = P.s4[k]; } break;
     default: for (int k = 0; k < 4; k++) { w[k] = P.c5[k]; w[5 + k] = P.s5[k]; } break;
+  }
+}
+
+// The same rows as weights of f(q) - f(0) for q = -5..-1, 1..5 (w[0..9] the
+// first derivative, w[10..19] the second), from the 5-term form: a first
+// derivative term W (f(P) - f(M)) adds W at P and -W at M, a second
+// derivative term W ((f(P) - f(0)) - (f(0) - f(M))) adds W at both.
+inline void row_dense(const double *w5, int row, double *w) {
+  for (int k = 0; k < 20; k++) w[k] = 0.0;
+  auto at = [](int q) { return q < 0 ? q + 5 : q + 4; };
+  constexpr RowOffsets ro = make_row_offsets();
+  auto off = [&](int e) { return (int)(signed char)((ro.w[row][e >> 2] >> (8 * (e & 3))) & 255); };
+  for (int k = 0; k < 5; k++) {
+    if (off(k)) w[at(off(k))] += w5[k];
+    if (off(5 + k)) w[at(off(5 + k))] -= w5[k];
+    if (off(10 + k)) w[10 + at(off(10 + k))] += w5[5 + k];
+    if (off(15 + k)) w[10 + at(off(15 + k))] += w5[5 + k];
   }
 }
 

@@ -405,8 +405,8 @@ class Solver:
         return bool(v.value)
 
     def set_tiles(self, narrow=(0, 0, 0)):
-        """Pass tiles per direction (0: rows of 32, 1: rows of 16); results do
-        not change."""
+        """Stores the tile flags; the passes have one tile shape, so neither
+        results nor speed change."""
         self._chk(self.lib.sg_set_tiles(self.h, (C.c_int * 3)(*narrow)))
 
     def tiles(self):
@@ -415,8 +415,8 @@ class Solver:
         return tuple(nw)
 
     def autotune(self, reps=5):
-        """Time the tile choices on the current state and keep the fastest;
-        returns (narrow, ms per substage of the tuned passes)."""
+        """Time the passes on the current state; returns (narrow, ms per
+        substage of the passes)."""
         ms = C.c_double(0)
         self._chk(self.lib.sg_autotune(self.h, int(reps), C.byref(ms)))
         return self.tiles(), ms.value
