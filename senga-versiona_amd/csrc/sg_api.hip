@@ -591,14 +591,15 @@ static int batch_capture(sg_batch *b) {
   hipGraph_t g = nullptr;
   if (hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal) != hipSuccess) return SG_EDEVICE;
   for (int r = 1; r <= 5; r++) {
-    if (b->L.inflow) launch_boundt(b->L, b->stream);
-    launch_prim(b->L, b->stream);
+    if (b->L.inflow && r == 1) launch_boundt(b->L, b->stream);
+    launch_prim(b->L, r - 1, b->stream);
     launch_pass(0, b->L, b->stream);
     if (b->L.radn) launch_radn(b->L, b->stream);
     launch_pass(1, b->L, b->stream);
     launch_pass(2, b->L, b->stream);
     if (b->L.bndx) launch_nscbc(b->L, b->stream);
-    launch_final(b->L, r, nullptr, b->stream);
+    if (r < 5) launch_cross(b->L, b->stream);   // LINCOM with the next launch_prim
+    else launch_final(b->L, r, nullptr, b->stream);
   }
   if (b->L.inflow) launch_bountt(b->L, b->stream);
   hipError_t e = hipStreamEndCapture(b->stream, &g);
@@ -906,12 +907,13 @@ int sg_set_timestep(sg_handle *h, double dt) {
   return refresh_member(h);
 }
 
-// BOUNDT .. BOUNDS (src/senga2.f:118-131): everything up to the register update.
-static int eval_rhs(sg_handle *h) {
+// BOUNDT .. BOUNDS (src/senga2.f:118-131): everything up to the register
+// update.  irk > 0: with the LINCOM of substage irk before it.
+static int eval_rhs(sg_handle *h, int irk) {
   const Launch &L = h->L;
   int rc = 0;
-  if (L.inflow) rc = timed(h, K_BOUNDT, [&] { launch_boundt(L, h->stream); });
-  if (!rc) rc = timed(h, K_PRIM, [&] { launch_prim(L, h->stream); });
+  if (L.inflow && !irk) rc = timed(h, K_BOUNDT, [&] { launch_boundt(L, h->stream); });
+  if (!rc) rc = timed(h, K_PRIM, [&] { launch_prim(L, irk, h->stream); });
   if (!rc) rc = timed(h, K_PASSX, [&] { launch_pass(0, L, h->stream); });
   if (!rc && L.radn) rc = timed(h, K_RADN, [&] { launch_radn(L, h->stream); });
   if (!rc && L.nblk[L_PASSY]) rc = timed(h, K_PASSY, [&] { launch_pass(1, L, h->stream); });
@@ -925,7 +927,7 @@ int sg_substage(sg_handle *h, int irk) {
   if (h->batch) return set_err(h, SG_ESTATE, "handle advances in a batch");
   if (!h->have_state) return set_err(h, SG_ESTATE, "no state uploaded");
   if (irk < 1 || irk > 5) return set_err(h, SG_EINVAL, "irk must be 1..5");
-  int rc = eval_rhs(h);
+  int rc = eval_rhs(h, 0);
   if (rc) return rc;
   return timed(h, K_FINAL, [&] { launch_final(h->L, irk, nullptr, h->stream); });
 }
@@ -1011,11 +1013,17 @@ int sg_get_timestep(sg_handle *h, double *tstep, double *errold, double *errldr)
 int sg_step(sg_handle *h, int nsteps) {
   if (!h) return SG_EINVAL;
   for (int n = 0; n < nsteps; n++) {
-    for (int r = 1; r <= 5; r++) {
-      int rc = sg_substage(h, r);
-      if (rc) return rc;
+    if (h->batch) return set_err(h, SG_ESTATE, "handle advances in a batch");
+    if (!h->have_state) return set_err(h, SG_ESTATE, "no state uploaded");
+    // sg_substage 1..5, the LINCOM of each substage done by the next one's
+    // point kernel; the step ends with both registers updated
+    int rc = 0;
+    for (int r = 1; r <= 5 && !rc; r++) {
+      rc = eval_rhs(h, r - 1);
+      if (!rc && r < 5) rc = timed(h, K_FINAL, [&] { launch_cross(h->L, h->stream); });
     }
-    int rc = sg_end_step(h);
+    if (!rc) rc = timed(h, K_FINAL, [&] { launch_final(h->L, 5, nullptr, h->stream); });
+    if (!rc) rc = sg_end_step(h);
     if (rc) return rc;
   }
   return 0;
@@ -1033,7 +1041,7 @@ int sg_rhs(sg_handle *h, int irk, double *rhs) {
   HIPCHK(h, hipMalloc((void **)&save, qbytes));
   HIPCHK(h, hipMalloc((void **)&out, qbytes));
   HIPCHK(h, hipMemcpyAsync(save, h->F.q, qbytes, hipMemcpyDeviceToDevice, h->stream));
-  int rc = eval_rhs(h);
+  int rc = eval_rhs(h, 0);
   if (!rc) rc = timed(h, K_FINAL, [&] { launch_final(h->L, 0, out, h->stream); });
   if (!rc) {
     size_t fb = sizeof(double) * P.npts;
@@ -1351,7 +1359,7 @@ int sg_autotune(sg_handle *h, int reps, double *ms) {
   int rc = snap_save(h, sn);
   if (rc) return rc;
   if (h->L.inflow) launch_boundt(h->L, h->stream);
-  launch_prim(h->L, h->stream);
+  launch_prim(h->L, 0, h->stream);
   double total = 0.0;
   for (int d = 0; d < 3; d++) total += time_launches(h->stream, reps, [&] { launch_pass(d, h->L, h->stream); });
   rc = snap_restore(h, sn, h->stream);
@@ -1385,7 +1393,7 @@ int sg_batch_autotune(sg_batch *b, int reps, double *ms) {
     if (!rc && hipStreamSynchronize(h->stream) != hipSuccess) rc = SG_EDEVICE;
   if (!rc) {
     if (b->L.inflow) launch_boundt(b->L, b->stream);
-    launch_prim(b->L, b->stream);
+    launch_prim(b->L, 0, b->stream);
   }
   double total = 0.0;
   for (int d = 0; d < 3 && !rc; d++)

@@ -12,7 +12,8 @@ namespace sg {
 template <int NS> void launch_tempin_t(const Params &, const sg_config *, const Fields &, hipStream_t);
 template <int NS> void launch_boundt_t(const Launch &, hipStream_t);
 template <int NS> void launch_bountt_t(const Launch &, hipStream_t);
-template <int NS> void launch_prim_t(const Launch &, hipStream_t);
+template <int NS> void launch_prim_t(const Launch &, int, hipStream_t);
+template <int NS> void launch_cross_t(const Launch &, hipStream_t);
 template <int NS> void launch_pass_t(int, const Launch &, hipStream_t);
 template <int NS> void launch_nscbc_t(const Launch &, hipStream_t);
 template <int NS> void launch_radn_t(const Launch &, hipStream_t);
@@ -49,9 +50,9 @@ void launch_bountt(const Launch &L, hipStream_t st) {
     default: break;
   }
 }
-void launch_prim(const Launch &L, hipStream_t st) {
+void launch_prim(const Launch &L, int irk, hipStream_t st) {
   switch (L.ns) {
-#define CASE(N) case N: launch_prim_t<N>(L, st); break;
+#define CASE(N) case N: launch_prim_t<N>(L, irk, st); break;
     SG_NS_LIST(CASE)
 #undef CASE
     default: break;
@@ -84,6 +85,14 @@ void launch_nscbc(const Launch &L, hipStream_t st) {
 void launch_final(const Launch &L, int irk, double *out, hipStream_t st) {
   switch (L.ns) {
 #define CASE(N) case N: launch_final_t<N>(L, irk, out, st); break;
+    SG_NS_LIST(CASE)
+#undef CASE
+    default: break;
+  }
+}
+void launch_cross(const Launch &L, hipStream_t st) {
+  switch (L.ns) {
+#define CASE(N) case N: launch_cross_t<N>(L, st); break;
     SG_NS_LIST(CASE)
 #undef CASE
     default: break;

@@ -142,7 +142,7 @@ inline __host__ __device__ int nface(int ns) { return face_corr(ns) + 5 + ns; }
 // that member's block b - blk0[kind].  A single case is a launch of one member.
 // L_FACE2: both x faces; L_PASSXE: the edge tiles of bounded x rows (the x
 // pass of a bounded x direction is two launches, interior and edge tiles)
-enum LaunchKind { L_FACE = 0, L_FACE2, L_POINT, L_PASSX, L_PASSY, L_PASSZ, L_FINAL, L_PASSXE, L_NKIND };
+enum LaunchKind { L_FACE = 0, L_FACE2, L_POINT, L_PASSX, L_PASSY, L_PASSZ, L_FINAL, L_PASSXE, L_CROSS, L_NKIND };
 
 struct Member {
   Params P;
@@ -178,7 +178,9 @@ void member_blocks(const Params &P, int nblk[L_NKIND]);
 // launchers (sg_kernels.hip)
 void launch_tempin(const Params &P, const sg_config *dcfg, const Fields &F, hipStream_t st);
 void launch_boundt(const Launch &L, hipStream_t st);
-void launch_prim(const Launch &L, hipStream_t st);
+// irk 0: the stage register as it is; irk 1..4: after the LINCOM of substage
+// irk from the accumulators (launch_cross before it), and BOUNDT
+void launch_prim(const Launch &L, int irk, hipStream_t st);
 void launch_pass(int dir, const Launch &L, hipStream_t st);
 // NSCBC face corrections (bounded x only), before launch_final
 void launch_nscbc(const Launch &L, hipStream_t st);
@@ -187,6 +189,9 @@ void launch_radn(const Launch &L, hipStream_t st);
 // substage irk (1..5): LINCOM for irk < 5, FINCOM for irk = 5, with each
 // member's coefficients; mode 2 (irk = 0): write the RHS to out instead
 void launch_final(const Launch &L, int irk, double *out, hipStream_t st);
+// the cross-direction terms of launch_final added to the accumulators, the
+// register update left to the next launch_prim
+void launch_cross(const Launch &L, hipStream_t st);
 // adaptive step: max over points and variables of |err|/(|run| + norm) into F.emax
 void launch_errmax(const Params &P, const Fields &F, hipStream_t st);
 void launch_zero(double *p, long n, hipStream_t st);

@@ -684,9 +684,67 @@ __device__ __forceinline__ void chem_step64(const M &m, int st, double t, double
   }
 }
 
-template <int NS, bool FIX>
+// LINCOM of substage irk (src/lincom.f:53-169) at one point, from the finished
+// right-hand sides in the accumulators, then BOUNDT (src/boundt.f:177-218) at
+// the inflow plane: the next substage's point kernel starts with it, so that
+// between the substages of a step no kernel of its own reads and writes both
+// registers (k_final moved 448 of its 608 B per point for them at 9 species).
+// v is the stage register's point; of it only density and momentum go to
+// memory here (the passes read them), the point kernels store the rest where
+// another kernel reads it.
+template <int NS, class R>
+__device__ __forceinline__ void lincom_point(const Params &P, const Fields &F, const Member &M, int irk, long idx,
+                                             double (&v)[5 + NS]) {
+  const long fs = P.fstride;
+  const uint32_t bo = (uint32_t)idx * 8u, br = (uint32_t)idx * (uint32_t)sizeof(R);
+  const R *A = (const R *)F.acc;
+  const double lhs = M.rkl[irk - 1], rhsc = M.rkr[irk - 1], erc = M.rke[irk - 1];
+  bool in = false;   // a point of the inflow plane, where all but the energy is imposed
+  if (P.inflow_xl) in = idx % P.nx == 0;
+  if (F.erk) {   // *ERR += RKERR * R, four variables at a time (each load would wait for the store before it)
+    for (int q0 = 0; q0 < 5 + NS; q0 += 4) {
+      double er[4];
+#pragma unroll
+      for (int q = 0; q < 4; q++)
+        if (q0 + q < 5 + NS) er[q] = fld(F.erk + (q0 + q) * fs, bo) + erc * (double)fld(A + (q0 + q) * fs, br);
+#pragma unroll
+      for (int q = 0; q < 4; q++)
+        if (q0 + q < 5 + NS && (q0 + q == 4 || !in)) fld(F.erk + (q0 + q) * fs, bo) = er[q];
+    }
+  }
+  SG_PHASE();
+  R rh[5 + NS];
+#pragma unroll
+  for (int q = 0; q < 5 + NS; q++) rh[q] = fld(A + q * fs, br);
+#pragma unroll
+  for (int q = 0; q < 5 + NS; q++) v[q] = fld(F.run + q * fs, bo);
+#pragma unroll
+  for (int q = 0; q < 5 + NS; q++) {
+    const double r = (double)rh[q], old = v[q];
+    if (q != 4 && in) {
+      v[q] = q == 0 ? P.drin : (q == 1 ? P.drin * P.uin : (q < 4 ? P.drin * 0.0 : P.drin * P.yrin[q < 5 ? 0 : q - 5]));
+    } else {
+      fld(F.run + q * fs, bo) = old + lhs * r;
+      v[q] = old + rhsc * r;
+    }
+  }
+#pragma unroll
+  for (int q = 0; q < 4; q++) fld(F.q + q * fs, bo) = v[q];
+}
+// the rest of the stage register, for the kernels that read it besides the point kernels
+template <int NS>
+__device__ __forceinline__ void store_stage(const Params &P, const Fields &F, uint32_t bo, double re,
+                                            const double (&ry)[NS]) {
+  fld(F.q + 4 * P.fstride, bo) = re;
+#pragma unroll
+  for (int s = 0; s < NS; s++) fld(F.q + (5 + s) * P.fstride, bo) = ry[s];
+}
+
+// UPD: the point kernel of a substage after the first, which begins with the
+// LINCOM of substage irk.
+template <int NS, bool FIX, bool UPD>
 __global__ void __launch_bounds__(BLK) __attribute__((amdgpu_waves_per_eu(4))) k_prim(const Member *__restrict__ mem,
-    const uint32_t *__restrict__ map, const sg_config *__restrict__ c, const Tables *__restrict__ tb) {
+    const uint32_t *__restrict__ map, const sg_config *__restrict__ c, const Tables *__restrict__ tb, int irk) {
   int lb;
   const Member &M = member_at<L_POINT>(mem, map, blockIdx.x, lb);
   const Params P = M.P;
@@ -701,11 +759,21 @@ __global__ void __launch_bounds__(BLK) __attribute__((amdgpu_waves_per_eu(4))) k
   const long fs = P.fstride;
   const double *q = F.q;
   double *pr = F.prim;
-  double d = fld(q, bo), ru = fld(q + fs, bo), rv = fld(q + 2 * fs, bo), rw = fld(q + 3 * fs, bo);
-  double re = fld(q + 4 * fs, bo);
+  // loaded before the update's stores, which they would otherwise wait for
+  const uint32_t idxo = fld(F.itndex, bo / 2u);
+  double t = fld(pr + P_T * fs, bo);
+  double st[5 + NS];
+  if constexpr (UPD) {
+    lincom_point<NS, double>(P, F, M, irk, idx, st);
+  } else {
+#pragma unroll
+    for (int v = 0; v < 5 + NS; v++) st[v] = fld(q + v * fs, bo);
+  }
+  const double d = st[0], ru = st[1], rv = st[2], rw = st[3], re = st[4];
   double ry[NS];
 #pragma unroll
-  for (int s = 0; s < NS; s++) ry[s] = fld(q + (5 + s) * fs, bo);
+  for (int s = 0; s < NS; s++) ry[s] = st[5 + s];
+  if (UPD && (P.radn || P.ltmask)) store_stage<NS>(P, F, bo, re, ry);
   // --- TEMPER (src/temper.f:58-160) ---
   const double ovd = 1.0 / d;   // one reciprocal for every division by rho
   double ukuk = (ru * ru + rv * rv + rw * rw) * ovd;
@@ -714,14 +782,12 @@ __global__ void __launch_bounds__(BLK) __attribute__((amdgpu_waves_per_eu(4))) k
 #pragma unroll
   for (int m = 1; m <= 5; m++) { tc[m] = 0.0; td[m] = 0.0; }
   double s7 = 0.0;
-  uint32_t idxo = fld(F.itndex, bo / 2u);
 #pragma unroll
   for (int s = 0; s < NS; s++) {
     temper_add(tb, s, itint_of(idxo, s), ry[s], tc, td);
     s7 = s7 + ry[s] * c->rgspec[s];
   }
   const double toltmp = (double)1.0e-10f;  // REAL literal, src/temper.f:33-34
-  double t = fld(pr + P_T * fs, bo);
   int iter = 1;
   bool ok = true;
   for (;;) {
@@ -1236,9 +1302,9 @@ __device__ __forceinline__ void chem_stepmx(const M &m, int st, float tf, double
 // exp2/log2 based intrinsics, except that the rate exponents (ln k = ln A +
 // n ln T - E/RT, Gibbs sums) are assembled in FP64 before the FP32
 // exponential, since they are differences of O(10..100) terms.
-template <int NS, bool FIX>
+template <int NS, bool FIX, bool UPD>
 __global__ void __launch_bounds__(BLK) __attribute__((amdgpu_waves_per_eu(4))) k_prim_mx(const Member *__restrict__ mem,
-    const uint32_t *__restrict__ map, const sg_config *__restrict__ c, const Tables *__restrict__ tb) {
+    const uint32_t *__restrict__ map, const sg_config *__restrict__ c, const Tables *__restrict__ tb, int irk) {
   int lb;
   const Member &M = member_at<L_POINT>(mem, map, blockIdx.x, lb);
   const Params P = M.P;
@@ -1249,11 +1315,20 @@ __global__ void __launch_bounds__(BLK) __attribute__((amdgpu_waves_per_eu(4))) k
   const long fs = P.fstride;
   const double *q = F.q;
   float *pr = (float *)F.prim;
-  double d = fld(q, bo), ru = fld(q + fs, bo), rv = fld(q + 2 * fs, bo), rw = fld(q + 3 * fs, bo);
-  double re = fld(q + 4 * fs, bo);
+  // loaded before the update's stores, which they would otherwise wait for
+  const uint32_t idxo = fld(F.itndex, bo / 2u);
+  double t = (double)fld(pr + P_T * fs, b4);
+  double st[5 + NS];
+  if constexpr (UPD) {
+    lincom_point<NS, float>(P, F, M, irk, idx, st);
+  } else {
+#pragma unroll
+    for (int v = 0; v < 5 + NS; v++) st[v] = fld(q + v * fs, bo);
+  }
+  const double d = st[0], ru = st[1], rv = st[2], rw = st[3], re = st[4];
   double ry[NS];
 #pragma unroll
-  for (int s = 0; s < NS; s++) ry[s] = fld(q + (5 + s) * fs, bo);
+  for (int s = 0; s < NS; s++) ry[s] = st[5 + s];
   // --- TEMPER (src/temper.f:58-160) ---
   const double ovd = 1.0 / d;   // one reciprocal for every division by rho
   double ukuk = (ru * ru + rv * rv + rw * rw) * ovd;
@@ -1262,14 +1337,12 @@ __global__ void __launch_bounds__(BLK) __attribute__((amdgpu_waves_per_eu(4))) k
 #pragma unroll
   for (int m = 1; m <= 5; m++) { tc[m] = 0.0; td[m] = 0.0; }
   double s7 = 0.0;
-  uint32_t idxo = fld(F.itndex, bo / 2u);
 #pragma unroll
   for (int s = 0; s < NS; s++) {
     temper_add(tb, s, itint_of(idxo, s), ry[s], tc, td);
     s7 = s7 + ry[s] * c->rgspec[s];
   }
   const double toltmp = (double)1.0e-10f;  // REAL literal, src/temper.f:33-34
-  double t = (double)fld(pr + P_T * fs, b4);
   int iter = 1;
   bool ok = true;
   for (;;) {
@@ -1310,6 +1383,10 @@ __global__ void __launch_bounds__(BLK) __attribute__((amdgpu_waves_per_eu(4))) k
   fld(F.itndex, bo / 2u) = nidx;
   SG_PHASE();
   double pres = t * s7;
+  if (UPD) {   // also where k_rate64 takes the stored temperature's rates
+    const double ts = (double)(float)t;
+    if (P.radn || P.ltmask || !(ts >= P.chlo && ts <= P.chhi)) store_stage<NS>(P, F, bo, re, ry);
+  }
   fld(pr + P_T * fs, b4) = (float)(t);
   fld(pr + P_P * fs, b4) = (float)(pres - P.pofs);
   // primitives
@@ -2455,21 +2532,33 @@ __global__ void __launch_bounds__(NSCBC_BLK) k_nscbc(const Member *__restrict__ 
 // face corrections (added; formed by k_nscbc) and the RK register update
 // (src/lincom.f:53-169, src/fincom.f:54-168).
 //
+// Between the substages of a step only the cross terms are formed here (CROSS)
+// and go back to the accumulators; the register update moves to the next
+// point kernel (lincom_point).  At 128^3 and 9 species that is 155 us in FP64
+// and 111 us mixed against 294 and 231 us with the update, while the point
+// kernel grows by 50 and 60 us; an RK step takes 6.74 -> 6.42 ms and 4.41 ->
+// 4.18 ms.
+//
 // A block owns an FX x FY x FZ tile of points, NPT per thread along z.  The
 // six mixed derivatives (d2u/dxdy, d2u/dxdz, d2v/dxdy, d2v/dydz, d2w/dxdz,
 // d2w/dydz) read their diagonal neighbours from u, v and w staged one at a
 // time into an LDS tile with a 5-deep halo in every direction (wrapped where
 // periodic, clamped where bounded), instead of 120 neighbour loads per point.
+template <bool BIG>
 struct FinalTile {
-  static constexpr int FX = 16, FY = 8, FZ = 4;
-  static constexpr int NPT = FX * FY * FZ / BLK;   // points per thread
-  static constexpr int ZS = BLK / (FX * FY);        // z stride between a thread's points
+  static constexpr int FX = 16, FY = 8, FZ = BIG ? 8 : 4;
+  static constexpr int NT = BIG ? 512 : 256;       // threads
+  static constexpr int NPT = FX * FY * FZ / NT;    // points per thread
+  static constexpr int ZS = NT / (FX * FY);        // z stride between a thread's points
   static constexpr int GX = FX + 10, GY = FY + 10, GZ = FZ + 10, GN = GX * GY * GZ;
 };
 
 // The per-point part of the final kernel at (i, j, k), given its six mixed
 // derivatives.
-template <bool BND, int NS, class R>
+// CROSS: the terms go back to the accumulators (the next substage's point
+// kernel does the register update); only momentum and energy have any, and
+// the x-face points their NSCBC corrections.
+template <bool BND, int NS, class R, bool CROSS>
 __device__ __forceinline__ void final_point(const Params &P, const Fields &F, const sg_config *__restrict__ c,
                                             int i, int j, int k, int mode, double lhs, double rhsc, double erc,
                                             double *__restrict__ out, R uxy, R vxy, R uxz, R wxz, R vyz, R wyz,
@@ -2482,8 +2571,8 @@ __device__ __forceinline__ void final_point(const Params &P, const Fields &F, co
   const R mu = fld(pr + P_MU * fs, bo);   // u, v, w come from the staged tile
   const R *G = (const R *)F.grad;
   auto gr = [&](int q) { return fld(G + q * fs, bo); };
-  const R *A = (const R *)F.acc;
-  R rD = fld(A, bo), rU = fld(A + fs, bo), rV = fld(A + 2 * fs, bo), rW = fld(A + 3 * fs, bo),
+  R *A = (R *)F.acc;
+  R rD = CROSS ? R(0) : fld(A, bo), rU = fld(A + fs, bo), rV = fld(A + 2 * fs, bo), rW = fld(A + 3 * fs, bo),
     rE = fld(A + 4 * fs, bo);
   auto fz = [&](const int *fl, int dir) {
     int m = dir == 0 ? i : (dir == 1 ? j : k);
@@ -2548,6 +2637,28 @@ __device__ __forceinline__ void final_point(const Params &P, const Fields &F, co
     t = fz(P.fvst, 1) ? R(0) : mu * ma + S7 * dmuy;
     rW = rW + t; rE = rE + w * t;
     rE = rE + mu * S7 * S7;
+  }
+  if constexpr (CROSS) {
+    if (BND && (i == 0 || i == P.nx - 1)) {   // NSCBC faces, as below
+      const long nf = (long)P.ny * P.nz, fq = (long)k * P.ny + j;
+      const double *cr = F.face + (i == 0 ? 0 : (long)nface(P.ns) * nf) + (long)face_corr(P.ns) * nf + fq;
+      rU = rU + (R)cr[nf];
+      rV = rV + (R)cr[2 * nf];
+      rW = rW + (R)cr[3 * nf];
+      rE = rE + (R)cr[4 * nf];
+      R a[1 + NS];   // every load before the first store
+      a[0] = fld(A, bo) + (R)cr[0];
+#pragma unroll
+      for (int s = 0; s < NS; s++) a[1 + s] = fld(A + (5 + s) * fs, bo) + (R)cr[(5 + s) * nf];
+      fld(A, bo) = a[0];
+#pragma unroll
+      for (int s = 0; s < NS; s++) fld(A + (5 + s) * fs, bo) = a[1 + s];
+    }
+    fld(A + fs, bo) = rU;
+    fld(A + 2 * fs, bo) = rV;
+    fld(A + 3 * fs, bo) = rW;
+    fld(A + 4 * fs, bo) = rE;
+    return;
   }
   R rY[NS];
 #pragma unroll
@@ -2630,13 +2741,14 @@ __device__ __forceinline__ void final_point(const Params &P, const Fields &F, co
   }
 }
 
-template <bool BND, int NS, class R>
-__global__ void __launch_bounds__(BLK) k_final(const Member *__restrict__ mem, const uint32_t *__restrict__ map,
-                                               const sg_config *__restrict__ c, int irk, double *__restrict__ out) {
-  using FT = FinalTile;
+template <bool BND, int NS, class R, bool CROSS, bool BIG>
+__global__ void __launch_bounds__(FinalTile<BIG>::NT) __attribute__((amdgpu_waves_per_eu(BIG ? 4 : 1))) k_final(
+    const Member *__restrict__ mem, const uint32_t *__restrict__ map, const sg_config *__restrict__ c, int irk,
+    double *__restrict__ out) {
+  using FT = FinalTile<BIG>;
   constexpr int FX = FT::FX, FY = FT::FY, FZ = FT::FZ, NPT = FT::NPT, GX = FT::GX, GY = FT::GY;
   int lb;
-  const Member &M = member_at<L_FINAL>(mem, map, xcd_block(blockIdx.x, gridDim.x), lb);
+  const Member &M = member_at<BIG ? L_CROSS : L_FINAL>(mem, map, xcd_block(blockIdx.x, gridDim.x), lb);
   const Params P = M.P;
   const Fields F = global_fields(M.F);
   // substage irk: LINCOM (mode 0) or FINCOM at the last substage (mode 1);
@@ -2683,34 +2795,56 @@ __global__ void __launch_bounds__(BLK) k_final(const Member *__restrict__ mem, c
     return g < n ? g : n - 1;
   };
   // staging: the tile is GX*GY columns of GZ values; thread t fetches
-  // columns t and t + BLK, all loads in flight at once, into registers and
-  // then stores them to LDS.  The next field's fetch is issued before the
-  // current field's derivatives are evaluated.  Column offsets are per
-  // thread, plane offsets are uniform.
-  constexpr int NCOL = GX * GY, GZ = FT::GZ;
-  static_assert(NCOL > BLK && NCOL <= 2 * BLK, "two columns per thread");
-  const bool col2 = t + BLK < NCOL;
-  auto coloff = [&](int cc) {
-    const int tx = cc % GX, ty = cc / GX;
-    return (uint32_t)(hidx(y0 - 5 + ty, ny, false) * nx + hidx(x0 - 5 + tx, nx, BND));
-  };
-  const uint32_t co0 = coloff(t), co1 = coloff(col2 ? t + BLK : t);
-  R stg[2][GZ];
-  auto fetch = [&](const R *f) {
+  // columns t, t + NT, all loads in flight at once, into registers and then
+  // stores them to LDS.  The next field's fetch is issued before the current
+  // field's derivatives are evaluated.  Column offsets are per thread, plane
+  // offsets are uniform.  Only what the field's stencils read is fetched: u
+  // the (x, y) and (x, z) planes of its points, v (x, y) and (y, z), w (x, z)
+  // and (y, z).
+  constexpr int NCOL = GX * GY, GZ = FT::GZ, NTH = FT::NT, NC = (NCOL + NTH - 1) / NTH;
+  uint32_t co[NC];
+  bool inx[NC], iny[NC];
 #pragma unroll
-    for (int z = 0; z < GZ; z++) {
+  for (int q = 0; q < NC; q++) {
+    const int cc = t + q * NTH, tx = cc % GX, ty = cc / GX;
+    const bool ok = cc < NCOL;
+    inx[q] = ok && tx >= 5 && tx < 5 + FX;
+    iny[q] = ok && ty >= 5 && ty < 5 + FY;
+    co[q] = ok ? (uint32_t)(hidx(y0 - 5 + ty, ny, false) * nx + hidx(x0 - 5 + tx, nx, BND)) : 0u;
+  }
+  R stg[NC][GZ];
+  auto columns = [&](auto field, auto f) {   // f(q, z) for the column values field 0, 1, 2 (u, v, w) needs
+    constexpr int FLD = decltype(field)::value;
+#pragma unroll
+    for (int q = 0; q < NC; q++) {
+      const bool halo = FLD == 0 ? iny[q] : (FLD == 1 ? inx[q] : inx[q] || iny[q]);   // z halo
+      const bool in = FLD == 2 ? halo : t + q * NTH < NCOL;
+      if (in) {
+#pragma unroll
+        for (int z = 5; z < 5 + FZ; z++) f(q, z);
+      }
+      if (halo) {
+#pragma unroll
+        for (int z = 0; z < 5; z++) {
+          f(q, z);
+          f(q, z + 5 + FZ);
+        }
+      }
+    }
+  };
+  auto fetch = [&](auto field) {
+    const R *f = pr + (P_U + decltype(field)::value) * fs;
+    columns(field, [&](int q, int z) {
       const uint32_t zo = (uint32_t)hidx(z0 - 5 + z, nz, false) * (uint32_t)(nx * ny);
-      stg[0][z] = fld(f, (zo + co0) * (uint32_t)sizeof(R));
-      if (col2) stg[1][z] = fld(f, (zo + co1) * (uint32_t)sizeof(R));
-    }
+      stg[q][z] = fld(f, (zo + co[q]) * (uint32_t)sizeof(R));
+    });
   };
-  auto store = [&]() {
-#pragma unroll
-    for (int z = 0; z < GZ; z++) {
-      tile[z * NCOL + t] = stg[0][z];
-      if (col2) tile[z * NCOL + t + BLK] = stg[1][z];
-    }
+  auto store = [&](auto field) {
+    columns(field, [&](int q, int z) { tile[z * NCOL + t + q * NTH] = stg[q][z]; });
   };
+  using FU = std::integral_constant<int, 0>;
+  using FV = std::integral_constant<int, 1>;
+  using FW = std::integral_constant<int, 2>;
   auto base = [&](int p) { return (lz0 + p * FT::ZS + 5) * GX * GY + (ly + 5) * GX + (lx + 5); };
   auto mix_x = [&](int B, int d2) {   // d2 = 1: (x, y); d2 = 2: (x, z)
     const int s2 = d2 == 1 ? GX : GX * GY;
@@ -2760,10 +2894,10 @@ __global__ void __launch_bounds__(BLK) k_final(const Member *__restrict__ mem, c
   // added in that order
   R uxy[NPT], uxz[NPT], vxy[NPT], vyz[NPT], wxz[NPT], wyz[NPT], uc[NPT], vc[NPT], wc[NPT];
   R dux[NPT], dvy[NPT], dwz[NPT], sxy[NPT], sxz[NPT], syz[NPT];
-  fetch(pr + P_U * fs);
-  store();
+  fetch(FU{});
+  store(FU{});
   __syncthreads();
-  fetch(pr + P_V * fs);
+  fetch(FV{});
 #pragma unroll
   for (int p = 0; p < NPT; p++) {
     uc[p] = tile[base(p)];
@@ -2776,9 +2910,9 @@ __global__ void __launch_bounds__(BLK) k_final(const Member *__restrict__ mem, c
     pin(dux[p]); pin(sxy[p]); pin(sxz[p]);
   }
   __syncthreads();
-  store();
+  store(FV{});
   __syncthreads();
-  fetch(pr + P_W * fs);
+  fetch(FW{});
 #pragma unroll
   for (int p = 0; p < NPT; p++) {
     vc[p] = tile[base(p)];
@@ -2791,7 +2925,7 @@ __global__ void __launch_bounds__(BLK) k_final(const Member *__restrict__ mem, c
     pin(sxy[p]); pin(dvy[p]); pin(syz[p]);
   }
   __syncthreads();
-  store();
+  store(FW{});
   __syncthreads();
 #pragma unroll
   for (int p = 0; p < NPT; p++) {
@@ -2808,7 +2942,7 @@ __global__ void __launch_bounds__(BLK) k_final(const Member *__restrict__ mem, c
   for (int p = 0; p < NPT; p++) {
     const int k = z0 + lz0 + p * FT::ZS;
     if (i < nx && j < ny && k < nz)
-      final_point<BND, NS, R>(P, F, c, i, j, k, mode, lhs, rhsc, erc, out, uxy[p], vxy[p], uxz[p], wxz[p],
+      final_point<BND, NS, R, CROSS>(P, F, c, i, j, k, mode, lhs, rhsc, erc, out, uxy[p], vxy[p], uxz[p], wxz[p],
                               vyz[p], wyz[p], uc[p], vc[p], wc[p], dux[p], dvy[p], dwz[p], sxy[p], sxz[p], syz[p]);
   }
 }
@@ -2855,22 +2989,26 @@ template <int NS>
 void launch_bountt_t(const Launch &L, hipStream_t st) {
   hipLaunchKernelGGL(k_bountt<NS>, dim3(L.nblk[L_FACE]), dim3(BLK), 0, st, L.mem, L.map[L_FACE]);
 }
-template <int NS>
-static void launch_prim_k(const Launch &L, hipStream_t st) {
+template <int NS, bool FIX, bool UPD>
+static void launch_prim_u(const Launch &L, int irk, hipStream_t st) {
   const dim3 g(L.nblk[L_POINT]), b(BLK);
-  if constexpr (NS == MechH2::nspec) {
-    if (L.mechfix) {
-      if (L.precision) hipLaunchKernelGGL((k_prim_mx<NS, true>), g, b, 0, st, L.mem, L.map[L_POINT], L.c, L.tab);
-      else hipLaunchKernelGGL((k_prim<NS, true>), g, b, 0, st, L.mem, L.map[L_POINT], L.c, L.tab);
-      return;
-    }
-  }
-  if (L.precision) hipLaunchKernelGGL((k_prim_mx<NS, false>), g, b, 0, st, L.mem, L.map[L_POINT], L.c, L.tab);
-  else hipLaunchKernelGGL((k_prim<NS, false>), g, b, 0, st, L.mem, L.map[L_POINT], L.c, L.tab);
+  const uint32_t *map = L.map[L_POINT];
+  if (L.precision) hipLaunchKernelGGL((k_prim_mx<NS, FIX, UPD>), g, b, 0, st, L.mem, map, L.c, L.tab, irk);
+  else hipLaunchKernelGGL((k_prim<NS, FIX, UPD>), g, b, 0, st, L.mem, map, L.c, L.tab, irk);
+}
+template <int NS, bool FIX>
+static void launch_prim_k(const Launch &L, int irk, hipStream_t st) {
+  if (irk) launch_prim_u<NS, FIX, true>(L, irk, st);
+  else launch_prim_u<NS, FIX, false>(L, 0, st);
 }
 template <int NS>
-void launch_prim_t(const Launch &L, hipStream_t st) {
-  launch_prim_k<NS>(L, st);
+void launch_prim_t(const Launch &L, int irk, hipStream_t st) {
+  bool fixed = false;
+  if constexpr (NS == MechH2::nspec) {
+    fixed = L.mechfix != 0;
+    if (fixed) launch_prim_k<NS, true>(L, irk, st);
+  }
+  if (!fixed) launch_prim_k<NS, false>(L, irk, st);
   if (L.precision) {   // mixed form: FP64 rates where FP32 cannot hold them
     const dim3 g(L.nblk[L_POINT]), b(BLK);
     bool fix = false;
@@ -2929,24 +3067,37 @@ void launch_radn_t(const Launch &L, hipStream_t st) {
   if (L.precision) hipLaunchKernelGGL((k_radn<NS, float>), g, b, 0, st, L.mem, L.map[L_POINT], L.c);
   else hipLaunchKernelGGL((k_radn<NS, double>), g, b, 0, st, L.mem, L.map[L_POINT], L.c);
 }
+template <int NS, bool CROSS, bool BIG>
+static void launch_final_c(const Launch &L, int irk, double *out, hipStream_t st) {
+  constexpr int K = BIG ? L_CROSS : L_FINAL;
+  const dim3 g(L.nblk[K]), b(FinalTile<BIG>::NT);
+  const uint32_t *map = L.map[K];
+  if (L.precision) {
+    if (L.bndx) hipLaunchKernelGGL((k_final<true, NS, float, CROSS, BIG>), g, b, 0, st, L.mem, map, L.c, irk, out);
+    else hipLaunchKernelGGL((k_final<false, NS, float, CROSS, BIG>), g, b, 0, st, L.mem, map, L.c, irk, out);
+  } else {
+    if (L.bndx) hipLaunchKernelGGL((k_final<true, NS, double, CROSS, BIG>), g, b, 0, st, L.mem, map, L.c, irk, out);
+    else hipLaunchKernelGGL((k_final<false, NS, double, CROSS, BIG>), g, b, 0, st, L.mem, map, L.c, irk, out);
+  }
+}
 template <int NS>
 void launch_final_t(const Launch &L, int irk, double *out, hipStream_t st) {
-  const dim3 g(L.nblk[L_FINAL]), b(BLK);
-  const uint32_t *map = L.map[L_FINAL];
-  if (L.precision) {
-    if (L.bndx) hipLaunchKernelGGL((k_final<true, NS, float>), g, b, 0, st, L.mem, map, L.c, irk, out);
-    else hipLaunchKernelGGL((k_final<false, NS, float>), g, b, 0, st, L.mem, map, L.c, irk, out);
-  } else {
-    if (L.bndx) hipLaunchKernelGGL((k_final<true, NS, double>), g, b, 0, st, L.mem, map, L.c, irk, out);
-    else hipLaunchKernelGGL((k_final<false, NS, double>), g, b, 0, st, L.mem, map, L.c, irk, out);
-  }
+  launch_final_c<NS, false, false>(L, irk, out, st);
+}
+// 16 x 8 x 8 tiles (half the halo of 16 x 8 x 4) once they fill the chip's 512
+// block slots; below that the smaller tiles finish earlier
+template <int NS>
+void launch_cross_t(const Launch &L, hipStream_t st) {
+  if (L.nblk[L_CROSS] >= 512) launch_final_c<NS, true, true>(L, 0, nullptr, st);
+  else launch_final_c<NS, true, false>(L, 0, nullptr, st);
 }
 
 #ifdef SG_NS
 template void launch_tempin_t<SG_NS>(const Params &, const sg_config *, const Fields &, hipStream_t);
 template void launch_boundt_t<SG_NS>(const Launch &, hipStream_t);
 template void launch_bountt_t<SG_NS>(const Launch &, hipStream_t);
-template void launch_prim_t<SG_NS>(const Launch &, hipStream_t);
+template void launch_prim_t<SG_NS>(const Launch &, int, hipStream_t);
+template void launch_cross_t<SG_NS>(const Launch &, hipStream_t);
 template void launch_pass_t<SG_NS>(int, const Launch &, hipStream_t);
 template void launch_nscbc_t<SG_NS>(const Launch &, hipStream_t);
 template void launch_radn_t<SG_NS>(const Launch &, hipStream_t);
@@ -2995,7 +3146,8 @@ void member_blocks(const Params &P, int nblk[L_NKIND]) {
   auto tiles = [&](int tx, int ty, int tz) {
     return ((P.nx + tx - 1) / tx) * ((P.ny + ty - 1) / ty) * ((P.nz + tz - 1) / tz);
   };
-  nblk[L_FINAL] = tiles(FinalTile::FX, FinalTile::FY, FinalTile::FZ);
+  nblk[L_FINAL] = tiles(FinalTile<false>::FX, FinalTile<false>::FY, FinalTile<false>::FZ);
+  nblk[L_CROSS] = tiles(FinalTile<true>::FX, FinalTile<true>::FY, FinalTile<true>::FZ);
   // passes: every tile of a row (periodic x), or the interior tiles of the
   // bounded rows (L_PASSX) and their edge tiles (L_PASSXE); y goes with x
   // where the launch has no transport options
