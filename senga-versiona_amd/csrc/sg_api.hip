@@ -165,6 +165,16 @@ static void build_tables(sg_config &c, Tables &t) {
       t.cpspecf[st][m] = (float)c.cpspec[st][m];
     }
   }
+  // the interval bound the two-interval species share
+  t.onebound = 1;
+  bool found = false;
+  t.tbound = 0.0;
+  for (int s = 0; s < c.nspec; s++) {
+    if (c.ntint[s] < 2) continue;
+    if (found && c.tinthi[s][0] != t.tbound) t.onebound = 0;
+    if (!found) t.tbound = c.tinthi[s][0];
+    found = true;
+  }
   t.diffsym = 1;
   for (int i = 0; i < c.nspec; i++)
     for (int j = i + 1; j < c.nspec; j++)

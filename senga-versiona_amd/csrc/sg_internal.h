@@ -79,6 +79,8 @@ struct Tables {
   double rgs[SG_MAX_SPEC];                       // species gas constants (RGSPEC), Dufour
   int diffsym;                                   // binary diffusion fits symmetric in (i, j)
   int ratedense;                                 // nuw is usable
+  int onebound;                                  // every two-interval species has the interval bound tbound
+  double tbound;
   // FP32 copies of the tables the mixed-precision kernels read, so that
   // uniform coefficients arrive as scalar FP32 loads instead of per-lane
   // FP64 -> FP32 conversions
