@@ -1641,8 +1641,9 @@ __global__ void __launch_bounds__(BLK) __attribute__((amdgpu_waves_per_eu(4))) k
 // LDS reads instead of 40), and three species a wave leave the registers for
 // both directions.  At 128^3 (9 species) the passes took 0.335 (x) + 0.285
 // (y) + 0.295 (z) ms in FP64 and 0.217 + 0.157 + 0.166 ms in FP32; x with y
-// now takes 0.44 and z 0.265 ms in FP64, 0.27 and 0.15 in FP32, the x-y pass
-// reading the primitives once (1305 -> 790 B per point of HBM traffic).
+// now takes 0.408 (0.272 interior, 0.136 edge tiles) and z 0.268 ms in FP64,
+// 0.250 and 0.148 in FP32, the x-y pass reading the primitives once (1305 ->
+// 790 B per point of HBM traffic).
 // Products with rho u_d (e rho u_d, Y rho u_d and the momentum fluxes rho u_d
 // u_b) are formed inside the stencils from two tiles.
 //
@@ -2024,17 +2025,26 @@ __attribute__((amdgpu_waves_per_eu(sizeof(R) == 8 ? 2 : (DX + (DV != 0) == 2 ? 3
   auto zf = [&](const int *flag, int dd) { return BND && dd == 0 && ((atL && flag[0]) || (atR && flag[1])); };
   // ADB zeroing of the correction-velocity divergence acts on the face planes
   const bool zadb_any = (i == 0 && P.fadb[0]) || (i == P.nx - 1 && P.fadb[1]);
-  // x-face point of an NSCBC case: copies of what the NSCBC kernel reads go
+  // x-face points of an NSCBC case: copies of what the NSCBC kernel reads go
   // to the face arrays (of the tiles of a bounded x direction only the edge
-  // tiles hold such points)
-  constexpr bool FACES = !DX || XP == 2;
-  auto facew = [&](int r) {
-    return FACES && active(r) && (P.inflow_xl || P.outflow_xr) && (i == 0 || i == P.nx - 1);
+  // tiles hold such points), a field's four points under one test.  (One test
+  // per value, and the chemical rates and pressure loaded where they were
+  // copied, cost 40 of the edge tiles' 164 us at 128^3; now 136 us.)  The test and the address are formed where they are used, so that they
+  // hold no registers through the pass.
+  auto face = [&]() {
+    return (!DX || XP == 2) && inx && (P.inflow_xl || P.outflow_xr) && (i == 0 || i == P.nx - 1);
   };
   const long fnf = (long)P.ny * P.nz;
-  auto fcw = [&](int slot, int r) -> double & {
+  auto face_at = [&](int slot, int r) -> double & {
     const int v = v0 + q4 + r, j = DV == 2 ? w0 : v, k = DV == 2 ? v : w0;
     return F.face[(i == 0 ? 0 : (long)nface(P.ns) * fnf) + (long)slot * fnf + (long)k * P.ny + j];
+  };
+  auto face_put = [&](int slot, const R (&val)[4]) {
+    if (face()) {
+#pragma unroll
+      for (int r = 0; r < 4; r++)
+        if (active(r)) face_at(slot, r) = (double)val[r];
+    }
   };
   __syncthreads();
   // the divergence of rho u, each row of the lanes' points by one wave
@@ -2115,44 +2125,46 @@ __attribute__((amdgpu_waves_per_eu(sizeof(R) == 8 ? 2 : (DX + (DV != 0) == 2 ? 3
   };
   if (wv == 0) {
     R hm0[4], ghm[ND][4];
-    // accumulator v of the hydrodynamic wave's point r; what a pass adds to is
-    // loaded before the stencils, so that no store waits for it
-    R oldh[RMW ? 5 : 1][4];
-    if (RMW) {
+    // accumulator v of point r; what a pass adds to is loaded a stage before,
+    // ahead of that stage's prefetch (loads return in order)
+    R o[4];
+    auto load_old = [&](int v) {
 #pragma unroll
-      for (int v = 0; v < 5; v++)
-#pragma unroll
-        for (int r = 0; r < 4; r++) oldh[RMW ? v : 0][r] = fld(A + (long)v * fs, pb(r));
-    }
-    auto add = [&](int v, int r, R x) { fld(A + (long)v * fs, pb(r)) = RMW ? oldh[RMW ? v : 0][r] + x : x; };
+      for (int r = 0; r < 4; r++) o[r] = RMW ? fld(A + (long)v * fs, pb(r)) : R(0);
+    };
+    auto add = [&](int v, int r, R x) { fld(A + (long)v * fs, pb(r)) = RMW ? o[r] + x : x; };
     // ---------------- hydrodynamic fields: mu, p, lambda, T, e, u, v, w, h_mix
-    R c[4], mu0[4], p0[4], dp[ND][4];
+    // Results leave for memory after the next put(), before the next loads go
+    // out: the wait for those loads would otherwise wait for the stores too.
+    R c[4], mu0[4], p0[4], dp[ND][4], dmu[ND][4];
     put(0);
     fetch_h(DEPTH);
     ders(W1{}, tb, mu0, [&](int dd, int r, R g1, R, R) {
-      if (active(r)) fld((R *)F.grad + (long)dir(dd) * fs, pb(r)) = g1;   // for the final kernel
+      dmu[dd][r] = g1;
+      pin(dmu[dd][r]);
     });
     // pressure, less PRUN(IPREF,JPREF,KPREF) (src/rhsvel.f:741)
     const R pref = pr[(long)P_P * fs];
 #pragma unroll
     for (int it = 0; it < NIT; it++) pf[1 % DEPTH][it] = pf[1 % DEPTH][it] - pref;
     put(1);
+#pragma unroll
+    for (int r = 0; r < 4; r++)
+      if (active(r)) {
+#pragma unroll
+        for (int dd = 0; dd < ND; dd++) fld((R *)F.grad + (long)dir(dd) * fs, pb(r)) = dmu[dd][r];   // for the final kernel
+      }
     fetch_h(1 + DEPTH);
     ders(W1{}, tb, p0, [&](int dd, int r, R g1, R, R) {
       dp[dd][r] = g1;
       pin(dp[dd][r]);
-      if (facew(r)) fcw(dir(dd) == 0 ? F_DPDX : (dir(dd) == 1 ? F_DPDY : F_DPDZ), r) = (double)g1;
     });
 #pragma unroll
-    for (int r = 0; r < 4; r++) {
-      if (DX && facew(r)) {
-        fcw(F_P, r) = (double)fld(pr + (long)P_P * fs, pb(r));
-        fcw(F_RHO, r) = fld(F.q, pb(r) * (uint32_t)(8 / sizeof(R)));
-      }
-      p0[r] = p0[r] + pref + (R)P.pofs;   // stored pressure is p - pofs
-    }
+    for (int r = 0; r < 4; r++) p0[r] = p0[r] + pref + (R)P.pofs;   // stored pressure is p - pofs
     // heat conduction (src/rhscal.f:427-797)
     put(2);
+#pragma unroll
+    for (int dd = 0; dd < ND; dd++) face_put(dir(dd) == 0 ? F_DPDX : (dir(dd) == 1 ? F_DPDY : F_DPDZ), dp[dd]);
     fetch_h(2 + DEPTH);
     {
       R lam[4], dl[ND][4];
@@ -2166,14 +2178,11 @@ __attribute__((amdgpu_waves_per_eu(sizeof(R) == 8 ? 2 : (DX + (DV != 0) == 2 ? 3
         aE[r] = aE[r] + dl[dd][r] * g1 + lam[r] * (zf(P.fcon, dd) ? R(0) : g2);
         pin(aE[r]);
       });
-      if (DX) {
-#pragma unroll
-        for (int r = 0; r < 4; r++)
-          if (facew(r)) fcw(F_T, r) = (double)c[r];
-      }
     }
     // continuity and energy convection (src/rhscal.f:141-415)
     put(4);
+    if (DX) face_put(F_T, c);
+    load_old(0);
     fetch_h(4 + DEPTH);
     ders(W14{}, tb, c, [&](int dd, int r, R g1, R, R gp) {
       aE[r] = aE[r] - R(0.5) * (gp + md0(dd, r) * g1);
@@ -2183,8 +2192,6 @@ __attribute__((amdgpu_waves_per_eu(sizeof(R) == 8 ? 2 : (DX + (DV != 0) == 2 ? 3
     for (int r = 0; r < 4; r++) {
       aE[r] = aE[r] - R(0.5) * c[r] * divm(r);
       pin(aE[r]);
-      if (DX && facew(r)) fcw(F_E, r) = (double)c[r];
-      if (active(r)) add(0, r, -divm(r));
     }
     // momentum: split convection from the resident rho u_d tiles and the
     // staged u_b (src/rhsvel.f:348-729, 1312-2110; the reference forms the
@@ -2192,12 +2199,31 @@ __attribute__((amdgpu_waves_per_eu(sizeof(R) == 8 ? 2 : (DX + (DV != 0) == 2 ? 3
     // same quantity, rounded differently in its last bit), pressure gradient
     // and work (src/rhsvel.f:741-917), separable viscous terms
     // (src/rhsvel.f:1462-2305)
+    R res[4], gx[ND][4];   // the component's right-hand side; its gradients (face copies)
+    auto face_of = [&](int a) {   // face copies of the stage before component a
+      if (a == 0) {
+        if (DX) face_put(F_E, c);
+        return;
+      }
+      if (DX) {
+        face_put(F_U + a - 1, c);
+        face_put(F_DUX + a - 1, gx[0]);
+      }
+      if (DV == 1 && a < 3) face_put(F_DUY + a - 1, gx[VD]);
+      if (DV == 2 && a != 2) face_put(a == 1 ? F_DUZ : F_DWZ, gx[VD]);
+    };
 #pragma unroll
     for (int a = 0; a < 3; a++) {
       R s[4], tv[4];
 #pragma unroll
       for (int r = 0; r < 4; r++) s[r] = tv[r] = R(0);
       put(5 + a);
+      // of the stage before: continuity, or the previous component's momentum
+#pragma unroll
+      for (int r = 0; r < 4; r++)
+        if (active(r)) add(a, r, a ? res[r] : -divm(r));
+      face_of(a);
+      load_old(1 + a);
       fetch_h(5 + a + DEPTH);
       ders(W124{}, tb, c, [&](int dd, int r, R g1, R g2, R gp) {
         const int d = dir(dd);
@@ -2210,21 +2236,25 @@ __attribute__((amdgpu_waves_per_eu(sizeof(R) == 8 ? 2 : (DX + (DV != 0) == 2 ? 3
           pin(aE[r]);
         }
         pin(s[r]); pin(tv[r]);
-        if (facew(r)) {
-          if (d == 0) fcw(F_DUX + a, r) = (double)g1;
-          if (d == 1 && a < 2) fcw(F_DUY + a, r) = (double)g1;
-          if (d == 2 && a != 1) fcw(a == 0 ? F_DUZ : F_DWZ, r) = (double)g1;
+        if (!DX || XP == 2) {
+          gx[dd][r] = g1;
+          pin(gx[dd][r]);
         }
       });
 #pragma unroll
       for (int r = 0; r < 4; r++) {
         aE[r] = aE[r] + tv[r] * c[r];
         pin(aE[r]);
-        if (active(r)) add(1 + a, r, s[r] + tv[r] - R(0.5) * c[r] * divm(r));
-        if (DX && facew(r)) fcw(F_U + a, r) = (double)c[r];
+        res[r] = s[r] + tv[r] - R(0.5) * c[r] * divm(r);
+        pin(res[r]);
       }
     }
     put(8);
+#pragma unroll
+    for (int r = 0; r < 4; r++)
+      if (active(r)) add(3, r, res[r]);
+    face_of(3);
+    load_old(4);
     ders(W1{}, tb, hm0, [&](int dd, int r, R g1, R, R) {
       ghm[dd][r] = zf(P.fdif, dd) || zf(P.fadb, dd) ? R(0) : g1;
       pin(ghm[dd][r]);
@@ -2241,7 +2271,8 @@ __attribute__((amdgpu_waves_per_eu(sizeof(R) == 8 ? 2 : (DX + (DV != 0) == 2 ? 3
       if (active(r)) add(4, r, aE[r]);
     }
   } else {
-    R aY[SPW][4], dYz[ND][SPW][4];
+    R aY[SPW][4], dYz[ND][SPW][4], hp[4];   // hp: the last species' enthalpy
+    constexpr bool LATE = sizeof(R) == 4;
     // ---------------- species (src/rhscal.f:1030-3944)
 #pragma unroll
     for (int q = 0; q < SPW; q++) {
@@ -2254,6 +2285,7 @@ __attribute__((amdgpu_waves_per_eu(sizeof(R) == 8 ? 2 : (DX + (DV != 0) == 2 ? 3
         for (int it = 0; it < NIT; it++) er[it] = pf[0][it];
       }
       put(3 * q);
+      if (DX && !EXT && LATE && q > 0) face_put(face_h(P.ns, sp - 1), hp);
       if (EXT) fetch(0, pr + prim_y(P, sp));
       else fetch_s(3 * q + DEPTH);
       ders(W1{}, tb, rd, [&](int dd, int r, R g1, R, R) {
@@ -2283,7 +2315,6 @@ __attribute__((amdgpu_waves_per_eu(sizeof(R) == 8 ? 2 : (DX + (DV != 0) == 2 ? 3
         dYz[dd][q][r] = g1;
         pin(aY[q][r]); pin(dif[r]); pin(dYz[dd][q][r]);
         if (BND) pin(dife[r]);
-        if (DX && dd == 0 && facew(r)) fcw(F_NSCAL + sp, r) = (double)g1;
       });
 #pragma unroll
       for (int r = 0; r < 4; r++) {
@@ -2291,12 +2322,17 @@ __attribute__((amdgpu_waves_per_eu(sizeof(R) == 8 ? 2 : (DX + (DV != 0) == 2 ? 3
         sum_at(1, r) += dif[r];
         if (!BND) dife[r] = dif[r];
         pin(aY[q][r]);
-        if (DX && facew(r)) {
-          fcw(face_y(P.ns, sp), r) = (double)c[r];
-          fcw(face_rate(P.ns, sp), r) = (double)fld((const R *)F.rate + (long)sp * fs, pb(r));
-        }
       }
+      // (FP64 has no registers to hold these until after the next put())
+      auto face_y0 = [&]() {
+        if (DX) {
+          face_put(F_NSCAL + sp, dYz[0][q]);
+          face_put(face_y(P.ns, sp), c);
+        }
+      };
+      if (!LATE) face_y0();
       put(3 * q + 2);
+      if (LATE) face_y0();
       const bool more = q + 1 < SPW && has(q + 1);
       const bool ltsp = EXT && ((P.ltmask >> sp) & 1u);
       if (EXT) {
@@ -2305,18 +2341,18 @@ __attribute__((amdgpu_waves_per_eu(sizeof(R) == 8 ? 2 : (DX + (DV != 0) == 2 ? 3
       } else {
         fetch_s(3 * q + 2 + DEPTH);
       }
-      R h[4];
+      R (&h)[4] = hp;
       if constexpr (!EXT) {
         ders(W1{}, tb, h, [&](int dd, int r, R g1, R, R) {
           const bool z = zf(P.fdif, dd) || zf(P.fadb, dd);
           aE[r] = aE[r] + ((z ? R(0) : g1) * dYz[dd][q][r]) * rd[r];
           pin(aE[r]);
         });
+        if (DX && !LATE) face_put(face_h(P.ns, sp), h);
 #pragma unroll
         for (int r = 0; r < 4; r++) {
           aE[r] = aE[r] + h[r] * dife[r];
           pin(aE[r]);
-          if (DX && facew(r)) fcw(face_h(P.ns, sp), r) = (double)h[r];
 #pragma unroll
           for (int dd = 0; dd < ND; dd++) dYz[dd][q][r] = zf(P.fdif, dd) ? R(0) : dYz[dd][q][r];
         }
@@ -2326,6 +2362,7 @@ __attribute__((amdgpu_waves_per_eu(sizeof(R) == 8 ? 2 : (DX + (DV != 0) == 2 ? 3
           dh[r] = g1;
           pin(dh[r]);
         });
+        if (DX) face_put(face_h(P.ns, sp), h);
         const bool zdif = zf(P.fdif, 0), zdifadb = zdif || zf(P.fadb, 0);
         // one transport option: flux s7 * grad(l), its derivative ds, with
         // the enthalpy ut and its derivative dut
@@ -2340,7 +2377,6 @@ __attribute__((amdgpu_waves_per_eu(sizeof(R) == 8 ? 2 : (DX + (DV != 0) == 2 ? 3
         };
 #pragma unroll
         for (int r = 0; r < 4; r++) {
-          if (DX && facew(r)) fcw(face_h(P.ns, sp), r) = (double)h[r];
           hu[r] = h[r];
           dhu[r] = dh[r];
           rdY[r] = rd[r] * c[r];
@@ -2435,6 +2471,8 @@ __attribute__((amdgpu_waves_per_eu(sizeof(R) == 8 ? 2 : (DX + (DV != 0) == 2 ? 3
 #pragma unroll
     for (int q = 0; q < SPW; q++) {
       if (!has(q)) break;
+      if (DX) face_put(face_rate(P.ns, s0 + q), old[q]);
+      if (DX && !EXT && LATE && (q + 1 == SPW || !has(q + 1))) face_put(face_h(P.ns, s0 + q), hp);
 #pragma unroll
       for (int r = 0; r < 4; r++) {
         R s = aY[q][r] - y0[q][r] * vt[r];
@@ -2486,7 +2524,7 @@ __global__ void __launch_bounds__(NSCBC_BLK) k_nscbc(const Member *__restrict__ 
   {
     const double strg = fc[F_CP * nf], strr = fc[F_RR * nf];
     const double strt = fv(F_T);
-    const double strd = fc[F_RHO * nf];
+    const double strd = F.q[idx];
     double gam1 = strg - strr;
     const double stre = fv(F_E) - gam1 * strt;
     gam1 = strr / gam1;
@@ -2523,7 +2561,7 @@ __global__ void __launch_bounds__(NSCBC_BLK) k_nscbc(const Member *__restrict__ 
     if (i == P.nx - 1 && P.outflow_xr) {
       // NSBCO1, src/bounds.f:1296-1458 (pointwise in/outflow switch and local-Mach beta off)
       const double bet = 0.050;
-      const double strp = (double)fv(F_P) + P.pofs;
+      const double strp = (double)((const R *)F.prim)[(long)P_P * P.fstride + idx] + P.pofs;
       const double t51 = -v * fc[F_DPDY * nf] - w * fc[F_DPDZ * nf];
       const double t52 = -strp * (dvy + dwz);
       const double t2b = -v * fv(F_DUY) - w * fv(F_DUZ);
