@@ -1677,9 +1677,12 @@ struct PassTile {
   static constexpr int ND = DX + (DV != 0);
   static constexpr int T = 16, NP = T * T;                 // points of the tile
   static constexpr int HX = DX ? 5 : 0, HV = DV ? 5 : 0;   // halo
-  // species a wave: what its registers hold (a direction more costs another
-  // value per species and point)
-  static constexpr int SPMAX = ND == 2 ? 3 : 4;
+  // species a wave: what its registers hold (a direction more, or the transport
+  // options, cost more values per species and point).  Three instead of four
+  // with the transport options: 16 species, 48^3, FP64 z 81 -> 69 us, y 81 ->
+  // 67, x 75 -> 64 and edge tiles 73 -> 58 us (7 waves instead of 5 a block, 6
+  // to 10 spilled registers instead of 16 to 35).
+  static constexpr int SPMAX = ND == 2 || EXT ? 3 : 4;
   static constexpr int NG = (NS + SPMAX - 1) / SPMAX;      // species waves
   static constexpr int SPW = (NS + NG - 1) / NG;
   static constexpr int NW = 1 + NG, NT = 64 * NW;
