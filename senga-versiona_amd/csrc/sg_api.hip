@@ -171,6 +171,7 @@ static void build_tables(sg_config &c, Tables &t) {
   t.tbound = 0.0;
   for (int s = 0; s < c.nspec; s++) {
     if (c.ntint[s] < 2) continue;
+    t.twomask |= 1u << s;
     if (found && c.tinthi[s][0] != t.tbound) t.onebound = 0;
     if (!found) t.tbound = c.tinthi[s][0];
     found = true;

@@ -81,6 +81,7 @@ struct Tables {
   int ratedense;                                 // nuw is usable
   int onebound;                                  // every two-interval species has the interval bound tbound
   double tbound;
+  uint32_t twomask;                              // the two-interval species, one bit each
   // FP32 copies of the tables the mixed-precision kernels read, so that
   // uniform coefficients arrive as scalar FP32 loads instead of per-lane
   // FP64 -> FP32 conversions

@@ -216,29 +216,21 @@ __device__ __forceinline__ double vmov_u(double c) {
   return r;
 }
 
-// The temperature interval it when every active lane of the wave holds the
-// same one, else -1; wave-uniform (from ballots), so the polynomials below
-// then run once with scalar coefficients.
-__device__ __forceinline__ int wave_interval(int it) {
-  const unsigned long long on = __ballot(it != 0), all = __ballot(1);
-  return __builtin_amdgcn_readfirstlane(on == 0ull ? 0 : (on == all ? 1 : -1));
+// the intervals of all species at temperature t, one bit each
+template <int NS>
+__device__ __forceinline__ uint32_t locate_all(const sg_config *c, const Tables *tb, double t) {
+  if (tb->onebound) return t > tb->tbound ? tb->twomask : 0u;
+  uint32_t n = 0;
+#pragma unroll
+  for (int s = 0; s < NS; s++) n += (uint32_t)locate(c, s, t) << s;
+  return n;
 }
 
-// Horner over the zero-padded SG_NCPMAX-term polynomial of interval it.
-// When the wave disagrees on it, both intervals are evaluated with uniform
-// (scalar) coefficients and the result is chosen per point, which is cheaper
-// than choosing every coefficient.  Both forms compute the same sums.  (The
-// enthalpy and Gibbs polynomials below keep the two-interval form only: with
-// the wave-uniform branch there too the FP64 point kernel spilled.)
+// Horner over the zero-padded SG_NCPMAX-term polynomial of interval it: both
+// intervals are evaluated with uniform (scalar) coefficients and the result is
+// chosen per point, which is cheaper than choosing every coefficient.
 __device__ __forceinline__ double horner(const double (&a)[SG_NTINT][SG_NCPMAX], int it, double x) {
   static_assert(SG_NTINT == 2, "two temperature intervals");
-  const int u = wave_interval(it);
-  if (u >= 0) {
-    double f = vmov_u(a[u][SG_NCPMAX - 1]);
-#pragma unroll
-    for (int m = SG_NCPMAX - 2; m >= 0; m--) f = fma_u(f, x, a[u][m]);
-    return f;
-  }
   double f0 = vmov_u(a[0][SG_NCPMAX - 1]), f1 = vmov_u(a[1][SG_NCPMAX - 1]);
 #pragma unroll
   for (int m = SG_NCPMAX - 2; m >= 0; m--) {
@@ -249,56 +241,44 @@ __device__ __forceinline__ double horner(const double (&a)[SG_NTINT][SG_NCPMAX],
 }
 
 // c(it) + x * poly(it)(x) for a two-interval table: formed for both intervals
-// with scalar coefficients and the result chosen per point (a choice of the
-// coefficients instead costs register copies and selects for every one).
-__device__ __forceinline__ double horner_c(const double (&a)[SG_NTINT][SG_NCPMAX], const double (&c0)[SG_NTINT],
-                                           int it, double x) {
-  double f0 = vmov_u(a[0][SG_NCPMAX - 1]), f1 = vmov_u(a[1][SG_NCPMAX - 1]);
+// with scalar coefficients (a: the two polynomials, c0: the two constants) and
+// the result chosen per point (a choice of the coefficients instead costs
+// register copies and selects for every one).
+__device__ __forceinline__ double horner_c(const double *a, const double *c0, int it, double x) {
+  double f0 = vmov_u(a[SG_NCPMAX - 1]), f1 = vmov_u(a[2 * SG_NCPMAX - 1]);
 #pragma unroll
   for (int m = SG_NCPMAX - 2; m >= 0; m--) {
-    f0 = fma_u(f0, x, a[0][m]);
-    f1 = fma_u(f1, x, a[1][m]);
+    f0 = fma_u(f0, x, a[m]);
+    f1 = fma_u(f1, x, a[SG_NCPMAX + m]);
   }
   f0 = fma_u(f0, x, c0[0]);
   f1 = fma_u(f1, x, c0[1]);
   return it ? f1 : f0;
 }
-// Gibbs function gbh(it)/T - gbs(it) ln T - poly(it)(T), both intervals formed,
-// one chosen (ovt = 1/T).
-__device__ __forceinline__ double gibbs_of(const Tables *tb, int s, int it, double t, double ovt, double lt) {
-  double f0 = vmov_u(tb->gb[s][0][SG_NCPMAX - 1]), f1 = vmov_u(tb->gb[s][1][SG_NCPMAX - 1]);
+// Gibbs function h(it)/T - s(it) ln T - poly(it)(T), both intervals formed, one
+// chosen (ovt = 1/T); a: the polynomials, hs: h(0), h(1), s(0), s(1).
+__device__ __forceinline__ double gibbs_of(const double *a, const double *hs, int it, double t, double ovt,
+                                           double lt) {
+  double f0 = vmov_u(a[SG_NCPMAX - 1]), f1 = vmov_u(a[2 * SG_NCPMAX - 1]);
 #pragma unroll
   for (int m = SG_NCPMAX - 2; m >= 0; m--) {
-    f0 = fma_u(f0, t, tb->gb[s][0][m]);
-    f1 = fma_u(f1, t, tb->gb[s][1][m]);
+    f0 = fma_u(f0, t, a[m]);
+    f1 = fma_u(f1, t, a[SG_NCPMAX + m]);
   }
-  const double g0 = tb->gbh[s][0] * ovt - tb->gbs[s][0] * lt - f0;
-  const double g1 = tb->gbh[s][1] * ovt - tb->gbs[s][1] * lt - f1;
+  const double g0 = hs[0] * ovt - hs[2] * lt - f0;
+  const double g1 = hs[1] * ovt - hs[3] * lt - f1;
   return it ? g1 : g0;
 }
 
 // TEMPER's polynomial sums (src/temper.f:92-128 with the coefficients of
 // src/chemin.f:906-916): species s of mass density y in interval it adds its
-// terms to tc (E(T) - E) and td (dE/dT).  A wave that agrees on it adds them
-// with that interval's scalar coefficients; otherwise y * c(interval) is
-// formed as y0 * c(0) + y1 * c(1) with exactly one of y0, y1 zero: the zero
-// term adds an exact zero, so every sum is the one formed with the chosen
-// interval alone, and the coefficients stay uniform.  Terms above the
-// interval's order add y * 0, which leaves the sums unchanged.
+// terms to tc (E(T) - E) and td (dE/dT).  Where the wave does not agree on the
+// intervals, y * c(interval) is formed as y0 * c(0) + y1 * c(1) with exactly
+// one of y0, y1 zero: the zero term adds an exact zero, so every sum is the one
+// formed with the chosen interval alone, and the coefficients stay uniform.
+// Terms above the interval's order add y * 0, which leaves the sums unchanged.
 __device__ __forceinline__ void temper_add(const Tables *tb, int s, int it, double y, double (&tc)[6],
                                            double (&td)[6]) {
-  const int u = wave_interval(it);
-  if (u >= 0) {
-    tc[0] = tc[0] + y * tb->hcp[s][u];
-    tc[1] = tc[1] + y * tb->ct[s][u][0];
-    td[1] = tc[1];
-#pragma unroll
-    for (int m = 2; m <= SG_NCPMAX; m++) {
-      tc[m] = tc[m] + y * tb->ct[s][u][m - 1];
-      td[m] = td[m] + y * tb->cp[s][u][m - 1];
-    }
-    return;
-  }
   const double y0 = it ? 0.0 : y, y1 = it ? y : 0.0;
   tc[0] = tc[0] + y0 * tb->hcp[s][0];
   tc[0] = tc[0] + y1 * tb->hcp[s][1];
@@ -312,6 +292,117 @@ __device__ __forceinline__ void temper_add(const Tables *tb, int s, int it, doub
     td[m] = td[m] + y0 * tb->cp[s][0][m - 1];
     td[m] = td[m] + y1 * tb->cp[s][1][m - 1];
   }
+}
+
+// Uniform coefficients, a group ahead.  Left to itself the compiler loads each
+// table entry right before its use and waits for it, 366 times in the point
+// kernel of 9 species; with 16 species the waves waited for two thirds of
+// their time.  pipe() runs use(k, coefficients of group k) for NG groups of up
+// to N values: the loads of the next group are issued before the group is
+// used, and held there.  With the transport fits in groups (exp_fits) and one
+// decision per wave on the temperature intervals, the point kernel between
+// substages takes 248 -> 214 us (16 species, 72x60x48), 85 -> 80 us (9
+// species, 93x71x57), 29 -> 26 us (24x20x21) and 363 -> 358 us at 128^3, where
+// HBM bounds it; mixed 235 -> 228 us, 69 -> 64 us (4-step methane, 96x80x64).
+template <int NG, int N, class T, class LOAD, class USE>
+__device__ __forceinline__ void pipe(LOAD load, USE use) {
+  T c[2][N];
+  load(0, c[0]);
+#pragma unroll
+  for (int g = 0; g < NG; g++) {
+    if (g + 1 < NG) {
+      load(g + 1, c[(g + 1) & 1]);
+      SG_PHASE();
+    }
+    use(g, c[g & 1]);
+    SG_PHASE();
+  }
+}
+
+// put(s, enthalpy) and put(s, Gibbs function) of every species at t
+template <int NS, class IT, class PUT>
+__device__ __forceinline__ void enthalpies(const Tables *tb, IT it, double t, PUT put) {
+  constexpr int N = 2 * SG_NCPMAX;
+  pipe<NS, N + 2, double>(
+      [&](int s, double (&c)[N + 2]) {
+#pragma unroll
+        for (int m = 0; m < N; m++) c[m] = tb->ch[s][m / SG_NCPMAX][m % SG_NCPMAX];
+        c[N] = tb->hch[s][0];
+        c[N + 1] = tb->hch[s][1];
+      },
+      [&](int s, const double (&c)[N + 2]) { put(s, horner_c(c, c + N, it(s), t)); });
+}
+template <int NS, class IT, class PUT>
+__device__ __forceinline__ void gibbs_all(const Tables *tb, IT it, double t, double ovt, double lt, PUT put) {
+  constexpr int N = 2 * SG_NCPMAX;
+  pipe<NS, N + 4, double>(
+      [&](int s, double (&c)[N + 4]) {
+#pragma unroll
+        for (int m = 0; m < N; m++) c[m] = tb->gb[s][m / SG_NCPMAX][m % SG_NCPMAX];
+#pragma unroll
+        for (int m = 0; m < 2; m++) {
+          c[N + m] = tb->gbh[s][m];
+          c[N + 2 + m] = tb->gbs[s][m];
+        }
+      },
+      [&](int s, const double (&c)[N + 4]) { put(s, gibbs_of(c, c + N, it(s), t, ovt, lt)); });
+}
+
+// The sums over all species; a wave whose points agree on every interval takes
+// each species' with that interval's scalar coefficients.
+template <int NS>
+__device__ __forceinline__ void temper_sums(const Tables *tb, uint32_t idxo, const double (&ry)[NS], double (&tc)[6],
+                                            double (&td)[6]) {
+  const uint32_t m0 = __builtin_amdgcn_readfirstlane(idxo);
+  if (__ballot(idxo != m0) == 0ull) {
+    pipe<NS, 10, double>(
+        [&](int s, double (&c)[10]) {
+          const int u = itint_of(m0, s);
+          c[0] = tb->hcp[s][u];
+#pragma unroll
+          for (int m = 0; m < 5; m++) c[1 + m] = tb->ct[s][u][m];
+#pragma unroll
+          for (int m = 1; m < 5; m++) c[5 + m] = tb->cp[s][u][m];
+        },
+        [&](int s, const double (&c)[10]) {
+          const double y = ry[s];
+          tc[0] = tc[0] + y * c[0];
+          tc[1] = tc[1] + y * c[1];
+          td[1] = tc[1];
+#pragma unroll
+          for (int m = 2; m <= SG_NCPMAX; m++) {
+            tc[m] = tc[m] + y * c[m];
+            td[m] = td[m] + y * c[4 + m];
+          }
+        });
+  } else {
+#pragma unroll
+    for (int s = 0; s < NS; s++) temper_add(tb, s, itint_of(idxo, s), ry[s], tc, td);
+  }
+}
+// rho cp = sum over the species of rho Y_k cp_k at the new intervals
+template <int NS>
+__device__ __forceinline__ double rho_cp(const Tables *tb, uint32_t nidx, const double (&ry)[NS], double t) {
+  double cp = 0.0;
+  const uint32_t m0 = __builtin_amdgcn_readfirstlane(nidx);
+  if (__ballot(nidx != m0) == 0ull) {
+    pipe<NS, 5, double>(
+        [&](int s, double (&c)[5]) {
+          const int u = itint_of(m0, s);
+#pragma unroll
+          for (int m = 0; m < 5; m++) c[m] = tb->cp[s][u][m];
+        },
+        [&](int s, const double (&c)[5]) {
+          double f = vmov_u(c[4]);
+#pragma unroll
+          for (int m = 3; m >= 0; m--) f = fma_u(f, t, c[m]);
+          cp = cp + ry[s] * f;
+        });
+  } else {
+#pragma unroll
+    for (int s = 0; s < NS; s++) cp = cp + ry[s] * horner(tb->cp[s], itint_of(nidx, s), t);
+  }
+  return cp;
 }
 
 // ---------------------------------------------------------------------------
@@ -476,23 +567,109 @@ __device__ __forceinline__ double trfit(const double *a, double x) {
 // NaN propagates.  13 VALU instructions and one LDS read, against ~22 for the
 // library exp.
 static constexpr double kExp2j[64] = {0x1.0000000000000p+0, 0x1.02c9a3e778061p+0, 0x1.059b0d3158574p+0, 0x1.0874518759bc8p+0, 0x1.0b5586cf9890fp+0, 0x1.0e3ec32d3d1a2p+0, 0x1.11301d0125b51p+0, 0x1.1429aaea92de0p+0, 0x1.172b83c7d517bp+0, 0x1.1a35beb6fcb75p+0, 0x1.1d4873168b9aap+0, 0x1.2063b88628cd6p+0, 0x1.2387a6e756238p+0, 0x1.26b4565e27cddp+0, 0x1.29e9df51fdee1p+0, 0x1.2d285a6e4030bp+0, 0x1.306fe0a31b715p+0, 0x1.33c08b26416ffp+0, 0x1.371a7373aa9cbp+0, 0x1.3a7db34e59ff7p+0, 0x1.3dea64c123422p+0, 0x1.4160a21f72e2ap+0, 0x1.44e086061892dp+0, 0x1.486a2b5c13cd0p+0, 0x1.4bfdad5362a27p+0, 0x1.4f9b2769d2ca7p+0, 0x1.5342b569d4f82p+0, 0x1.56f4736b527dap+0, 0x1.5ab07dd485429p+0, 0x1.5e76f15ad2148p+0, 0x1.6247eb03a5585p+0, 0x1.6623882552225p+0, 0x1.6a09e667f3bcdp+0, 0x1.6dfb23c651a2fp+0, 0x1.71f75e8ec5f74p+0, 0x1.75feb564267c9p+0, 0x1.7a11473eb0187p+0, 0x1.7e2f336cf4e62p+0, 0x1.82589994cce13p+0, 0x1.868d99b4492edp+0, 0x1.8ace5422aa0dbp+0, 0x1.8f1ae99157736p+0, 0x1.93737b0cdc5e5p+0, 0x1.97d829fde4e50p+0, 0x1.9c49182a3f090p+0, 0x1.a0c667b5de565p+0, 0x1.a5503b23e255dp+0, 0x1.a9e6b5579fdbfp+0, 0x1.ae89f995ad3adp+0, 0x1.b33a2b84f15fbp+0, 0x1.b7f76f2fb5e47p+0, 0x1.bcc1e904bc1d2p+0, 0x1.c199bdd85529cp+0, 0x1.c67f12e57d14bp+0, 0x1.cb720dcef9069p+0, 0x1.d072d4a07897cp+0, 0x1.d5818dcfba487p+0, 0x1.da9e603db3285p+0, 0x1.dfc97337b9b5fp+0, 0x1.e502ee78b3ff6p+0, 0x1.ea4afa2a490dap+0, 0x1.efa1bee615a27p+0, 0x1.f50765b6e4540p+0, 0x1.fa7c1819e90d8p+0};
+struct ExpT {
+  double r, tj;
+  int ni;
+  // the reduction and the table read; value() the rest
+  __device__ __forceinline__ void start(double x, const double *xt) {
+    const double INV = 0x1.71547652b82fep+6, L1 = 0x1.62e42ff000000p-7, L2 = -0x1.718432a1b0e26p-41;
+    // n = nearest integer to x*64/ln2 by the shifter 1.5*2^52: the fused sum
+    // rounds to an integer, whose low 32 bits are n (two's complement)
+    const double SH = 0x1.8p52;
+    const double tsh = __builtin_fma(x, INV, SH);
+    const double n = tsh - SH;
+    ni = (int)(unsigned)__builtin_bit_cast(unsigned long long, tsh);
+    tj = xt[ni & 63];
+    r = __builtin_fma(-n, L1, x);
+    r = __builtin_fma(-n, L2, r);
+  }
+  __device__ __forceinline__ double value() const {
+    double q = __builtin_fma(r, 1.0 / 120.0, 1.0 / 24.0);
+    q = __builtin_fma(q, r, 1.0 / 6.0);
+    q = __builtin_fma(q, r, 0.5);
+    const double p = __builtin_fma(q, r * r, r);
+    return __builtin_ldexp(__builtin_fma(tj, p, tj), ni >> 6);
+  }
+};
 __device__ __forceinline__ double exp_t(double x, const double *xt) {
-  const double INV = 0x1.71547652b82fep+6, L1 = 0x1.62e42ff000000p-7, L2 = -0x1.718432a1b0e26p-41;
-  // n = nearest integer to x*64/ln2 by the shifter 1.5*2^52: the fused sum
-  // rounds to an integer, whose low 32 bits are n (two's complement)
-  const double SH = 0x1.8p52;
-  const double tsh = __builtin_fma(x, INV, SH);
-  const double n = tsh - SH;
-  const int ni = (int)(unsigned)__builtin_bit_cast(unsigned long long, tsh);
-  double r = __builtin_fma(-n, L1, x);
-  r = __builtin_fma(-n, L2, r);
-  double q = __builtin_fma(r, 1.0 / 120.0, 1.0 / 24.0);
-  q = __builtin_fma(q, r, 1.0 / 6.0);
-  q = __builtin_fma(q, r, 0.5);
-  const double p = __builtin_fma(q, r * r, r);
-  const double tj = xt[ni & 63];
-  return __builtin_ldexp(__builtin_fma(tj, p, tj), ni >> 6);
+  ExpT e;
+  e.start(x, xt);
+  return e.value();
 }
+
+// put(i, exp(pre(fit_i(x)))) for the N transport fits at row(i), four at a time:
+// their table reads are issued together, and the next four fits' coefficients
+// arrive while this group's polynomials are evaluated.
+template <int N, class ROW, class PRE, class PUT>
+__device__ __forceinline__ void exp_fits(double x, const double *xt, ROW row, PRE pre, PUT put) {
+  constexpr int G = 4;
+  double c[2][G][SG_NTRC];
+  auto load = [&](int g) {
+#pragma unroll
+    for (int i = 0; i < G; i++)
+      if (g * G + i < N) {
+        const double *a = row(g * G + i);
+#pragma unroll
+        for (int m = 0; m < SG_NTRC; m++) c[g & 1][i][m] = a[m];
+      }
+  };
+  load(0);
+#pragma unroll
+  for (int g = 0; g < (N + G - 1) / G; g++) {
+    ExpT e[G];
+#pragma unroll
+    for (int i = 0; i < G; i++)
+      if (g * G + i < N) e[i].start(pre(trfit(c[g & 1][i], x)), xt);
+    SG_PHASE();
+    if ((g + 1) * G < N) load(g + 1);
+    SG_PHASE();
+#pragma unroll
+    for (int i = 0; i < G; i++)
+      if (g * G + i < N) put(g * G + i, e[i].value());
+    SG_PHASE();
+  }
+}
+// the same in FP32, where the exponential reads no table: put(i, fit_i(x)),
+// eight fits' coefficients ahead
+template <int N, class ROW, class PUT>
+__device__ __forceinline__ void fits_f(float x, ROW row, PUT put) {
+  constexpr int G = 8;
+  pipe<(N + G - 1) / G, G * SG_NTRC, float>(
+      [&](int g, float (&c)[G * SG_NTRC]) {
+#pragma unroll
+        for (int i = 0; i < G; i++)
+          if (g * G + i < N) {
+            const float *a = row(g * G + i);
+#pragma unroll
+            for (int m = 0; m < SG_NTRC; m++) c[i * SG_NTRC + m] = a[m];
+          }
+      },
+      [&](int g, const float (&c)[G * SG_NTRC]) {
+#pragma unroll
+        for (int i = 0; i < G; i++)
+          if (g * G + i < N) {
+            float f = c[i * SG_NTRC + SG_NTRC - 1];
+#pragma unroll
+            for (int m = SG_NTRC - 2; m >= 0; m--) f = fma_u(f, x, c[i * SG_NTRC + m]);
+            put(g * G + i, f);
+          }
+      });
+}
+// the species pairs a < b, row by row
+template <int NS>
+struct Pairs {
+  int a[NS * (NS - 1) / 2 + 1] = {}, b[NS * (NS - 1) / 2 + 1] = {};
+  constexpr Pairs() {
+    int p = 0;
+    for (int i = 0; i < NS; i++)
+      for (int j = i + 1; j < NS; j++, p++) {
+        a[p] = i;
+        b[p] = j;
+      }
+  }
+};
+template <int NS>
+__constant__ constexpr Pairs<NS> kPairs{};
 
 // ---------------------------------------------------------------------------
 // CHRATE step loop (src/chrate.f:146-760), shared by the two sources of
@@ -807,12 +984,10 @@ __global__ void __launch_bounds__(BLK) __attribute__((amdgpu_waves_per_eu(4))) k
   tc[0] = 0.5 * ukuk - re;
 #pragma unroll
   for (int m = 1; m <= 5; m++) { tc[m] = 0.0; td[m] = 0.0; }
+  temper_sums<NS>(tb, idxo, ry, tc, td);
   double s7 = 0.0;
 #pragma unroll
-  for (int s = 0; s < NS; s++) {
-    temper_add(tb, s, itint_of(idxo, s), ry[s], tc, td);
-    s7 = s7 + ry[s] * c->rgspec[s];
-  }
+  for (int s = 0; s < NS; s++) s7 = s7 + ry[s] * c->rgspec[s];
   const double toltmp = (double)1.0e-10f;  // REAL literal, src/temper.f:33-34
   int iter = 1;
   bool ok = true;
@@ -840,17 +1015,8 @@ __global__ void __launch_bounds__(BLK) __attribute__((amdgpu_waves_per_eu(4))) k
     coords(P, idx, i, j, k);
     set_error(F.err, SG_ETEMPER, i, j, k);
   }
-  uint32_t nidx = 0;
-  double cp = 0.0;
-  int itn[NS];
-#pragma unroll
-  for (int s = 0; s < NS; s++) {
-    int it = locate(c, s, t);
-    itn[s] = it;
-    nidx += (uint32_t)it << s;
-    cp = cp + ry[s] * horner(tb->cp[s], it, t);
-  }
-  cp = cp * ovd;
+  const uint32_t nidx = locate_all<NS>(c, tb, t);
+  const double cp = rho_cp<NS>(tb, nidx, ry, t) * ovd;
   fld(F.itndex, bo / 2u) = nidx;
   SG_PHASE();
   double pres = t * s7;
@@ -872,12 +1038,11 @@ __global__ void __launch_bounds__(BLK) __attribute__((amdgpu_waves_per_eu(4))) k
     // the divisions X_k / lambda_k share one (batch_recip; a few ulp from the
     // reference's quotients)
     double c1 = 0.0, c2 = 0.0, c3 = 0.0, ictr[NS];
-#pragma unroll
-    for (int s = 0; s < NS; s++) {
-      const double ctr = exp_t(trfit(c->condco[s], transp), xt);
-      ictr[s] = ctr;
-      c1 = c1 + (ry[s] * c->ovwmol[s]) * ctr;
-    }
+    exp_fits<NS>(transp, xt, [&](int s) { return c->condco[s]; }, [](double f) { return f; },
+                 [&](int s, double ctr) {
+                   ictr[s] = ctr;
+                   c1 = c1 + (ry[s] * c->ovwmol[s]) * ctr;
+                 });
     batch_recip<NS>(ictr);
 #pragma unroll
     for (int s = 0; s < NS; s++) {
@@ -909,11 +1074,7 @@ __global__ void __launch_bounds__(BLK) __attribute__((amdgpu_waves_per_eu(4))) k
     // Gibbs functions of all species at this temperature, each formed as
     // src/chrate.f:612-632 forms it for every step it enters
     double gibbs[NS];
-#pragma unroll
-    for (int s = 0; s < NS; s++) {
-      int it = itn[s];
-      gibbs[s] = gibbs_of(tb, s, it, t, ovt, lt);
-    }
+    gibbs_all<NS>(tb, [&](int s) { return itint_of(nidx, s); }, t, ovt, lt, [&](int s, double g) { gibbs[s] = g; });
     if constexpr (FIX) {
       using MT = CtMech<MechH2>;
       double cy[NS];
@@ -948,14 +1109,11 @@ __global__ void __launch_bounds__(BLK) __attribute__((amdgpu_waves_per_eu(4))) k
 #pragma unroll
   for (int s = 0; s < NS; s++) y[s] = ry[s] * ovd;
   double hmix = 0.0;
-#pragma unroll
-  for (int s = 0; s < NS; s++) {
+  enthalpies<NS>(tb, [&](int s) { return itint_of(nidx, s); }, t, [&](int s, double h) {
     fld(pr + prim_y(P, s), bo) = y[s];
-    int it = itn[s];
-    double h = horner_c(tb->ch[s], tb->hch[s], it, t);
     fld(pr + prim_h(P, s), bo) = h;
     hmix = hmix + h * y[s];
-  }
+  });
   fld(pr + P_HMIX * fs, bo) = hmix;
   SG_PHASE();
   if (!P.mixavg) {
@@ -986,15 +1144,13 @@ __global__ void __launch_bounds__(BLK) __attribute__((amdgpu_waves_per_eu(4))) k
       double cs[NS];
 #pragma unroll
       for (int s = 0; s < NS; s++) cs[s] = 0.0;
-#pragma unroll
-      for (int a = 0; a < NS; a++) {
-#pragma unroll
-        for (int b = a + 1; b < NS; b++) {
-          const double ictd = exp_t(-trfit(c->diffco[a][b], transp), xt);
-          cs[a] = cs[a] + yw2p[b] * ictd;
-          cs[b] = cs[b] + yw2p[a] * ictd;
-        }
-      }
+      exp_fits<NS * (NS - 1) / 2>(transp, xt, [&](int p) { return c->diffco[kPairs<NS>.a[p]][kPairs<NS>.b[p]]; },
+                                  [](double f) { return -f; },
+                                  [&](int p, double ictd) {
+                                    const int a = kPairs<NS>.a[p], b = kPairs<NS>.b[p];
+                                    cs[a] = cs[a] + yw2p[b] * ictd;
+                                    cs[b] = cs[b] + yw2p[a] * ictd;
+                                  });
       double c2[NS];
 #pragma unroll
       for (int s = 0; s < NS; s++) c2[s] = cs[s] * wmomix;
@@ -1030,28 +1186,41 @@ __global__ void __launch_bounds__(BLK) __attribute__((amdgpu_waves_per_eu(4))) k
     // reciprocals 1/sqrt(mu_j) share one division, and so do the divisions
     // mu_s / sum_s (batch_recip).
     double mus[NS], sq[NS], rsq[NS], yw[NS];
+    exp_fits<NS>(transp, xt, [&](int s) { return c->viscco[s]; }, [](double f) { return 0.5 * f; },
+                 [&](int s, double v) {
+                   sq[s] = v;
+                   rsq[s] = v;
+                   mus[s] = v * v;
+                 });
 #pragma unroll
-    for (int s = 0; s < NS; s++) {
-      const double hf = 0.5 * trfit(c->viscco[s], transp);
-      sq[s] = exp_t(hf, xt);
-      rsq[s] = sq[s];
-      mus[s] = sq[s] * sq[s];
-      yw[s] = y[s] * c->ovwmol[s];
-    }
+    for (int s = 0; s < NS; s++) yw[s] = y[s] * c->ovwmol[s];
     batch_recip<NS>(rsq);
     double c1 = 0.0, wc2[NS];
 #pragma unroll
-    for (int s = 0; s < NS; s++) {
-      double c2 = 0.0;
+    for (int s = 0; s < NS; s++) wc2[s] = 0.0;
+    pipe<(NS * NS + 7) / 8, 16, double>(
+        [&](int g, double (&w)[16]) {
 #pragma unroll
-      for (int js = 0; js < NS; js++) {
-        double fornow = js == s ? 1.0 : sq[s] * rsq[js];
-        fornow = 1.0 + fornow * c->wilko2[s][js];
-        fornow = c->wilko1[s][js] * fornow * fornow;
-        c2 = c2 + yw[js] * fornow;
-      }
-      wc2[s] = c2;
-    }
+          for (int i = 0; i < 8; i++) {
+            const int k = g * 8 + i;
+            if (k < NS * NS) {
+              w[i] = c->wilko2[k / NS][k % NS];
+              w[8 + i] = c->wilko1[k / NS][k % NS];
+            }
+          }
+        },
+        [&](int g, const double (&w)[16]) {
+#pragma unroll
+          for (int i = 0; i < 8; i++) {
+            const int k = g * 8 + i, s = k / NS, js = k % NS;
+            if (k < NS * NS) {
+              double fornow = js == s ? 1.0 : sq[s] * rsq[js];
+              fornow = 1.0 + fornow * w[i];
+              fornow = w[8 + i] * fornow * fornow;
+              wc2[s] = wc2[s] + yw[js] * fornow;
+            }
+          }
+        });
     batch_recip<NS>(wc2);
 #pragma unroll
     for (int s = 0; s < NS; s++) c1 = c1 + yw[s] * (mus[s] * wc2[s]);
@@ -1099,10 +1268,8 @@ __global__ void __launch_bounds__(BLK) k_rate64(const Member *__restrict__ mem, 
   const double lt = log(t), ovt = 1.0 / t;
   double gibbs[NS], rate[NS];
 #pragma unroll
-  for (int s = 0; s < NS; s++) {
-    gibbs[s] = gibbs_of(tb, s, locate(c, s, t), t, ovt, lt);
-    rate[s] = 0.0;
-  }
+  for (int s = 0; s < NS; s++) rate[s] = 0.0;
+  gibbs_all<NS>(tb, [&](int s) { return locate(c, s, t); }, t, ovt, lt, [&](int s, double g) { gibbs[s] = g; });
   auto ex = [](double x) { return exp(x); };
   if constexpr (FIX) {
     using MT = CtMech<MechH2>;
@@ -1362,12 +1529,10 @@ __global__ void __launch_bounds__(BLK) __attribute__((amdgpu_waves_per_eu(4))) k
   tc[0] = 0.5 * ukuk - re;
 #pragma unroll
   for (int m = 1; m <= 5; m++) { tc[m] = 0.0; td[m] = 0.0; }
+  temper_sums<NS>(tb, idxo, ry, tc, td);
   double s7 = 0.0;
 #pragma unroll
-  for (int s = 0; s < NS; s++) {
-    temper_add(tb, s, itint_of(idxo, s), ry[s], tc, td);
-    s7 = s7 + ry[s] * c->rgspec[s];
-  }
+  for (int s = 0; s < NS; s++) s7 = s7 + ry[s] * c->rgspec[s];
   const double toltmp = (double)1.0e-10f;  // REAL literal, src/temper.f:33-34
   int iter = 1;
   bool ok = true;
@@ -1395,17 +1560,8 @@ __global__ void __launch_bounds__(BLK) __attribute__((amdgpu_waves_per_eu(4))) k
     coords(P, idx, i, j, k);
     set_error(F.err, SG_ETEMPER, i, j, k);
   }
-  uint32_t nidx = 0;
-  double cp = 0.0;
-  int itn[NS];
-#pragma unroll
-  for (int s = 0; s < NS; s++) {
-    int it = locate(c, s, t);
-    itn[s] = it;
-    nidx += (uint32_t)it << s;
-    cp = cp + ry[s] * horner(tb->cp[s], it, t);
-  }
-  cp = cp * ovd;
+  const uint32_t nidx = locate_all<NS>(c, tb, t);
+  const double cp = rho_cp<NS>(tb, nidx, ry, t) * ovd;
   fld(F.itndex, bo / 2u) = nidx;
   SG_PHASE();
   double pres = t * s7;
@@ -1435,17 +1591,13 @@ __global__ void __launch_bounds__(BLK) __attribute__((amdgpu_waves_per_eu(4))) k
   if (P.mixavg) {
     transp = __logf(tf * (float)(1.0 / P.tdifgb));
     float c1 = 0.0f, c2 = 0.0f, c3 = 0.0f;
-#pragma unroll
-    for (int s = 0; s < NS; s++) {
-      float f = tb->condf[s][SG_NTRC - 1];
-#pragma unroll
-      for (int m = SG_NTRC - 2; m >= 0; m--) f = fma_u(f, transp, tb->condf[s][m]);
+    fits_f<NS>(transp, [&](int s) { return tb->condf[s]; }, [&](int s, float f) {
       float ctr = __expf(f);
       float fornow = ryf[s] * tb->ovwf[s];
       c1 = c1 + fornow * ctr;
       c2 = c2 + qf(fornow, ctr);
       c3 = c3 + fornow;
-    }
+    });
     c3 = rf(c3);
     c1 = c1 * c3;
     c2 = c2 * c3;
@@ -1473,11 +1625,7 @@ __global__ void __launch_bounds__(BLK) __attribute__((amdgpu_waves_per_eu(4))) k
     for (int s = 0; s < NS; s++) rate[s] = 0.0f;
     const double lt = log(t), ovt = 1.0 / t;
     double gibbs[NS];
-#pragma unroll
-    for (int s = 0; s < NS; s++) {
-      int it = itn[s];
-      gibbs[s] = gibbs_of(tb, s, it, t, ovt, lt);
-    }
+    gibbs_all<NS>(tb, [&](int s) { return itint_of(nidx, s); }, t, ovt, lt, [&](int s, double g) { gibbs[s] = g; });
     if constexpr (FIX) {
       using MT = CtMech<MechH2>;
       float cy[NS];
@@ -1508,16 +1656,13 @@ __global__ void __launch_bounds__(BLK) __attribute__((amdgpu_waves_per_eu(4))) k
   // --- mass fractions and enthalpies (src/rhscal.f:1444-1470), FP64, stored FP32 ---
   float y[NS];
   double hmix = 0.0;
-#pragma unroll
-  for (int s = 0; s < NS; s++) {
+  enthalpies<NS>(tb, [&](int s) { return itint_of(nidx, s); }, t, [&](int s, double h) {
     const double yd = ry[s] * ovd;
     y[s] = (float)yd;
     fld(pr + prim_y(P, s), b4) = y[s];
-    int it = itn[s];
-    double h = horner_c(tb->ch[s], tb->hch[s], it, t);
     fld(pr + prim_h(P, s), b4) = (float)h;
     hmix = hmix + h * yd;
-  }
+  });
   fld(pr + P_HMIX * fs, b4) = (float)hmix;
   SG_PHASE();
   if (!P.mixavg) {
@@ -1551,15 +1696,13 @@ __global__ void __launch_bounds__(BLK) __attribute__((amdgpu_waves_per_eu(4))) k
         cs[s] = 0.0f;
         yw2p[s] = yw2[s] * ppd;
       }
-#pragma unroll
-      for (int a = 0; a < NS; a++) {
-#pragma unroll
-        for (int b = a + 1; b < NS; b++) {
-          const float ictd = __expf(-fit(tb->difff[a][b]));
-          cs[a] = cs[a] + yw2p[b] * ictd;
-          cs[b] = cs[b] + yw2p[a] * ictd;
-        }
-      }
+      fits_f<NS * (NS - 1) / 2>(transp, [&](int p) { return tb->difff[kPairs<NS>.a[p]][kPairs<NS>.b[p]]; },
+                                [&](int p, float f) {
+                                  const int a = kPairs<NS>.a[p], b = kPairs<NS>.b[p];
+                                  const float ictd = __expf(-f);
+                                  cs[a] = cs[a] + yw2p[b] * ictd;
+                                  cs[b] = cs[b] + yw2p[a] * ictd;
+                                });
 #pragma unroll
       for (int s = 0; s < NS; s++) {
         float c1 = c1t - yt[s];
@@ -1584,26 +1727,37 @@ __global__ void __launch_bounds__(BLK) __attribute__((amdgpu_waves_per_eu(4))) k
     SG_PHASE();
     // Wilke viscosity (src/rhscal.f:3854-3891), FP32
     float mus[NS], sq[NS], rsq[NS], yw[NS];
-#pragma unroll
-    for (int s = 0; s < NS; s++) {
-      mus[s] = __expf(fit(tb->viscf[s]));
+    fits_f<NS>(transp, [&](int s) { return tb->viscf[s]; }, [&](int s, float f) {
+      mus[s] = __expf(f);
       sq[s] = __builtin_amdgcn_sqrtf(mus[s]);
       rsq[s] = rf(sq[s]);
       yw[s] = y[s] * tb->ovwf[s];
-    }
-    float c1 = 0.0f;
+    });
+    float c1 = 0.0f, c2 = 0.0f;
+    pipe<(NS * NS + 15) / 16, 32, float>(
+        [&](int g, float (&w)[32]) {
 #pragma unroll
-    for (int s = 0; s < NS; s++) {
-      float c2 = 0.0f;
+          for (int i = 0; i < 16; i++) {
+            const int k = g * 16 + i;
+            if (k < NS * NS) {
+              w[i] = tb->wilk2f[k / NS][k % NS];
+              w[16 + i] = tb->wilk1f[k / NS][k % NS];
+            }
+          }
+        },
+        [&](int g, const float (&w)[32]) {
 #pragma unroll
-      for (int js = 0; js < NS; js++) {
-        float fornow = js == s ? 1.0f : sq[s] * rsq[js];
-        fornow = 1.0f + fornow * tb->wilk2f[s][js];
-        fornow = tb->wilk1f[s][js] * fornow * fornow;
-        c2 = c2 + yw[js] * fornow;
-      }
-      c1 = c1 + yw[s] * qf(mus[s], c2);
-    }
+          for (int i = 0; i < 16; i++) {
+            const int k = g * 16 + i, s = k / NS, js = k % NS;
+            if (k < NS * NS) {
+              float fornow = js == s ? 1.0f : sq[s] * rsq[js];
+              fornow = 1.0f + fornow * w[i];
+              fornow = w[16 + i] * fornow * fornow;
+              c2 = js ? c2 + yw[js] * fornow : yw[js] * fornow;
+              if (js == NS - 1) c1 = c1 + yw[s] * qf(mus[s], c2);
+            }
+          }
+        });
     fld(pr + P_MU * fs, b4) = c1;
   }
   // face data for NSCBC: cp and mixture gas constant (src/rhscal.f:72-131)
