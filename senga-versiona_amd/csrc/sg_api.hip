@@ -156,7 +156,10 @@ static void build_tables(sg_config &c, Tables &t) {
     }
   }
   for (int b = 0; b < SG_MAX_BODY; b++)
-    for (int s = 0; s < SG_MAX_SPEC; s++) t.effyf[b][s] = (float)c.effy3b[b][s];
+    for (int s = 0; s < SG_MAX_SPEC; s++) {
+      t.effw[b][s] = c.ovwmol[s] * c.effy3b[b][s];
+      t.effwf[b][s] = t.ovwf[s] * (float)c.effy3b[b][s];
+    }
   for (int st = 0; st < SG_MAX_STEP; st++) {
     for (int s = 0; s < SG_MAX_SPEC; s++) t.nuwf[st][s] = (float)t.nuw[st][s];
     for (int m = 0; m < SG_MAX_SSL; m++) {
@@ -164,6 +167,25 @@ static void build_tables(sg_config &c, Tables &t) {
       t.crspecf[st][m] = (float)c.crspec[st][m];
       t.cpspecf[st][m] = (float)c.cpspec[st][m];
     }
+  }
+  for (int st = 0; st < c.nstep; st++) {
+    StepRec &r = t.step[st];
+    auto b4 = [](int b0, int b1, int b2, int b3) {
+      return (uint32_t)b0 | (uint32_t)b1 << 8 | (uint32_t)b2 << 16 | (uint32_t)b3 << 24;
+    };
+    r.kind = b4(c.mblist[st], c.mglist[st] != 0, c.mllist[st], c.mtlist[st]);
+    r.len = b4(c.mslist[st], c.nsslen[st], c.nrslen[st], c.npslen[st]);
+    r.frac = b4(c.nrclen[st], c.npclen[st], 0, 0);
+    auto spec = [&](const int32_t *list, int len, int q) { return q < len ? (int)list[q] : c.nspec; };
+    auto four = [&](const int32_t *l, int n, int q) {
+      return b4(spec(l, n, q), spec(l, n, q + 1), spec(l, n, q + 2), spec(l, n, q + 3));
+    };
+    r.rs = four(c.nrspec[st], c.nrslen[st], 0);
+    r.ps = four(c.npspec[st], c.npslen[st], 0);
+    r.ss[0] = four(c.nsspec[st], c.nsslen[st], 0);
+    r.ss[1] = four(c.nsspec[st], c.nsslen[st], 4);
+    for (int q = 0; q < 3; q++) r.rp[q] = c.rparam[st][q];
+    for (int q = 0; q < SG_NALL; q++) r.dmu[q] = q < c.nsslen[st] ? c.diffmu[st][q] : 0.0;
   }
   // the interval bound the two-interval species share
   t.onebound = 1;

@@ -60,6 +60,23 @@ struct Params {
 // kernels evaluate them with fixed trip counts and uniform loads.
 #define SG_NCPMAX 5   // highest cp order the temperature solve accepts (src/temper.f NCTMAX)
 #define SG_NROW 11    // derivative row kinds: interior, 5 left and 5 right closure rows
+// One reaction step of a mechanism read at run time, packed: kinds and list
+// lengths, the first SG_NFWD reactants and products and the first SG_NALL
+// species with their stoichiometric differences (longer lists go on in
+// sg_config), filled up with the index nspec, whose concentration reads 1 and
+// whose Gibbs function reads 0.
+#define SG_NFWD 4
+#define SG_NALL 6
+struct StepRec {
+  uint32_t kind;    // bytes: third body, reversible, Lindemann, Troe
+  uint32_t len;     // bytes: SRI; lengths of the species, reactant and product lists
+  uint32_t frac;    // bytes: lengths of the fractional-order lists (forward, reverse)
+  uint32_t rs, ps;  // reactants, products
+  uint32_t ss[2];   // species
+  uint32_t pad;
+  double rp[3];
+  double dmu[SG_NALL];
+};
 struct Tables {
   double roww[SG_NROW][10];                      // 5-term row weights W1, W2 per row kind
   double rowd[SG_NROW][20];                      // the same rows as weights of f(q) - f(0), q = -5..-1, 1..5: first, second
@@ -81,6 +98,9 @@ struct Tables {
   int ratedense;                                 // nuw is usable
   int onebound;                                  // every two-interval species has the interval bound tbound
   double tbound;
+  StepRec step[SG_MAX_STEP + 1];
+  double effw[SG_MAX_BODY][SG_MAX_SPEC];         // ovwmol * effy3b
+  float effwf[SG_MAX_BODY][SG_MAX_SPEC];         // the product of the FP32 copies
   uint32_t twomask;                              // the two-interval species, one bit each
   // FP32 copies of the tables the mixed-precision kernels read, so that
   // uniform coefficients arrive as scalar FP32 loads instead of per-lane
@@ -89,7 +109,6 @@ struct Tables {
   float condf[SG_MAX_SPEC][SG_NTRC], viscf[SG_MAX_SPEC][SG_NTRC];
   float difff[SG_MAX_SPEC][SG_MAX_SPEC][SG_NTRC];
   float wilk1f[SG_MAX_SPEC][SG_MAX_SPEC], wilk2f[SG_MAX_SPEC][SG_MAX_SPEC];
-  float effyf[SG_MAX_BODY][SG_MAX_SPEC];
   float nuwf[SG_MAX_STEP][SG_MAX_SPEC];
   float diffmwf[SG_MAX_STEP][SG_MAX_SSL], crspecf[SG_MAX_STEP][SG_MAX_SSL], cpspecf[SG_MAX_STEP][SG_MAX_SSL];
 };
