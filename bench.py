@@ -69,21 +69,25 @@ def kernel_bytes(name, ns, bounded, nx=128):
     """Algorithmic bytes per grid point of one launch: each distinct input
     field read once and each output written once (FP64 fields, 4-byte index).
     The face kernels touch the nx = 1 and nx = n planes only: their bytes are
-    spread over the grid (divided by nx)."""
+    spread over the grid (divided by nx).  prim and final: the mean over the
+    five launches of a step, of which four of prim begin with the register
+    update and four of final only add the cross terms."""
     f = 8
     nprim = 9 + 3 * ns
     if name in ("boundt", "bountt"):   # inflow values of 5+N fields at x-left
         return f * (5 + ns) / nx
     if name == "nscbc":                # face data (6+N) + stage register (5+N) + corrections (5+N), two faces
         return 2 * f * ((6 + ns) + 2 * (5 + ns)) / nx
-    if name == "prim":          # reads stage (5+N), T, index; writes primitives, rate, index
-        return f * (5 + ns + 1) + 4 + f * (nprim + ns) + 4
-    if name == "pass_x":        # rho, 3 momenta, primitives, rate -> accumulators, d mu/dx
-        return f * (4 + nprim + ns) + f * (5 + ns) + f
+    if name == "prim":          # reads stage (5+N), T, index; writes primitives, rate, index;
+        io = f + 4 + f * (nprim + ns) + 4   # after an update: accumulators, run (r/w), 4 stage fields (w) for the stage
+        return (f * (5 + ns) + io + 4 * (3 * f * (5 + ns) + 4 * f + io)) / 5
+    if name == "pass_x":        # x with y: rho, 3 momenta, primitives, rate -> accumulators, d mu/dx, d mu/dy
+        return f * (4 + nprim + ns) + f * (5 + ns) + 2 * f
     if name in ("pass_y", "pass_z"):   # accumulators read-modify-write
         return f * (4 + nprim) + 2 * f * (5 + ns) + f
-    if name == "final":         # accumulators, 3 viscosity gradients, u,v,w,mu, run (r/w), stage (w)
-        return f * (5 + ns) + f * 3 + f * 4 + 2 * f * (5 + ns) + f * (5 + ns)
+    if name == "final":         # 3 viscosity gradients, u,v,w,mu; accumulators, run (r/w), stage (w), or
+        io = f * 3 + f * 4      # momentum and energy accumulators (r/w)
+        return (io + f * (5 + ns) + 2 * f * (5 + ns) + f * (5 + ns) + 4 * (io + 8 * f)) / 5
     return 0
 
 
