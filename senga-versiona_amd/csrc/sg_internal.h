@@ -63,8 +63,8 @@ struct Params {
 // One reaction step of a mechanism read at run time, packed: kinds and list
 // lengths, the first SG_NFWD reactants and products and the first SG_NALL
 // species with their stoichiometric differences (longer lists go on in
-// sg_config), filled up with the index nspec, whose concentration reads 1 and
-// whose Gibbs function reads 0.
+// sg_config), filled up with the index nspec, which stands for a concentration
+// of 1 and a Gibbs function of weight 0.
 #define SG_NFWD 4
 #define SG_NALL 6
 struct StepRec {

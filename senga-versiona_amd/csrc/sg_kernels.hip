@@ -689,7 +689,32 @@ __constant__ constexpr Pairs<NS> kPairs{};
 // dependent loads per entry, the point kernel took 216 instead of 198 us (16
 // species, 35 steps, 72x60x48) and 65 instead of 56.5 us (8 species, 4 steps
 // of fractional orders, mixed, 96x80x64).
-template <int NS>
+//
+// A step's lists index a point's concentrations and Gibbs functions in LDS, one
+// row of BLK values per species, and these rows decide how many blocks share a
+// CU.  The fill-up entries read a row of ones and a row of zeros more, where
+// that leaves as many blocks (fill_rows 2); else the species list's, whose
+// weights are 0, read species 0 (1), or the reactants' and products' too, a 1
+// being chosen in their place (0).  At 64^3, point kernel: 9 species in FP64
+// with both rows have three blocks a CU and take 104 us, four blocks and 78 us
+// with one; 13 species mixed 101 and 72 us.  Where no block is at stake the
+// rows are the cheaper form: 16 species in FP64 220 us with either, 237 with
+// none; 12 species 136 with both, 138 with one.
+template <class T>
+constexpr int list_blocks(int nc, int ng) {   // blocks of a CU, at most four (k_prim also holds exp_t's table)
+  const int n = 163840 / (BLK * (nc * (int)sizeof(T) + ng * 8) + (sizeof(T) == 8 ? 512 : 0));
+  return n < 4 ? n : 4;
+}
+template <int NS, class T>
+constexpr int fill_rows = list_blocks<T>(NS + 1, NS + 1) == list_blocks<T>(NS, NS) ? 2
+                          : list_blocks<T>(NS + 1, NS) == list_blocks<T>(NS, NS) ? 1 : 0;
+// rows of the two arrays
+template <int NS, class T>
+constexpr int rows_c = NS + (fill_rows<NS, T> > 0);
+template <int NS, class T>
+constexpr int rows_g = NS + (fill_rows<NS, T> > 1);
+
+template <int NS, int ROWS>
 struct RtMech {
   const sg_config *c;
   const Tables *tb;
@@ -700,9 +725,14 @@ struct RtMech {
   __device__ T conc(T s1, uint32_t list, int len, const int32_t (&all)[SG_MAX_SSL], CY cyv) const {
     T v[SG_NFWD];
 #pragma unroll
-    for (int q = 0; q < SG_NFWD; q++) v[q] = cyv(byte(list, q));
+    for (int q = 0; q < SG_NFWD; q++) {
+      const int s = byte(list, q);
+      v[q] = cyv(ROWS > 0 || s < NS ? s : 0);
+    }
 #pragma unroll
-    for (int q = 0; q < SG_NFWD; q++) s1 = s1 * (v[q] > T(0) ? v[q] : T(0));
+    for (int q = 0; q < SG_NFWD; q++)
+      if constexpr (ROWS > 0) s1 = s1 * (v[q] > T(0) ? v[q] : T(0));
+      else s1 = s1 * (q < len ? (v[q] > T(0) ? v[q] : T(0)) : T(1));
 #pragma unroll 1
     for (int q = SG_NFWD; q < len; q++) {
       const T x = cyv(all[q]);
@@ -722,7 +752,10 @@ struct RtMech {
   __device__ double gsum(int st, double s2, GB gbv) const {
     double v[SG_NALL];
 #pragma unroll
-    for (int q = 0; q < SG_NALL; q++) v[q] = gbv(byte(r.ss[q / 4], q % 4));
+    for (int q = 0; q < SG_NALL; q++) {
+      const int s = byte(r.ss[q / 4], q % 4);
+      v[q] = gbv(ROWS > 1 || s < NS ? s : 0);
+    }
 #pragma unroll
     for (int q = 0; q < SG_NALL; q++) s2 = s2 + r.dmu[q] * v[q];
 #pragma unroll 1
@@ -1154,16 +1187,16 @@ __global__ void __launch_bounds__(BLK) __attribute__((amdgpu_waves_per_eu(4))) k
       // Molar concentrations and Gibbs functions of this point in LDS, so
       // that a step's species lists (uniform, known only at run time) index
       // them with one LDS read instead of a select over all species.
-      __shared__ double lcy[NS + 1][BLK], lgb[NS + 1][BLK];
+      __shared__ double lcy[rows_c<NS, double>][BLK], lgb[rows_g<NS, double>][BLK];
       const int tl = threadIdx.x;
-      lcy[NS][tl] = 1;   // what the lists are filled up with
-      lgb[NS][tl] = 0;
+      if constexpr (rows_c<NS, double> > NS) lcy[NS][tl] = 1;
+      if constexpr (rows_g<NS, double> > NS) lgb[NS][tl] = 0;
 #pragma unroll
       for (int s = 0; s < NS; s++) {
         lcy[s][tl] = ry[s] * c->ovwmol[s];
         lgb[s][tl] = gibbs[s];
       }
-      RtMech<NS> mr{c, tb};
+      RtMech<NS, fill_rows<NS, double>> mr{c, tb};
       for_steps(mr, [&](int st) {
         chem_step64<NS>(mr, st, t, lt, ovt, ry, [&](int s) { return lcy[s][tl]; }, [&](int s) { return lgb[s][tl]; },
                         rate, [&](double x) { return exp_t(x, xt); });
@@ -1349,16 +1382,16 @@ __global__ void __launch_bounds__(BLK) k_rate64(const Member *__restrict__ mem, 
   } else {
     // species lists index the point's values at run time: from LDS, one
     // slot per thread (as in k_prim)
-    __shared__ double lcy[NS + 1][BLK], lgb[NS + 1][BLK];
+    __shared__ double lcy[rows_c<NS, double>][BLK], lgb[rows_g<NS, double>][BLK];
     const int tl = threadIdx.x;
-    lcy[NS][tl] = 1.0;   // what the lists are filled up with
-    lgb[NS][tl] = 0.0;
+    if constexpr (rows_c<NS, double> > NS) lcy[NS][tl] = 1.0;
+    if constexpr (rows_g<NS, double> > NS) lgb[NS][tl] = 0.0;
 #pragma unroll
     for (int s = 0; s < NS; s++) {
       lcy[s][tl] = ry[s] * c->ovwmol[s];
       lgb[s][tl] = gibbs[s];
     }
-    RtMech<NS> mr{c, tb};
+    RtMech<NS, fill_rows<NS, double>> mr{c, tb};
     for_steps(mr, [&](int st) {
       chem_step64<NS>(mr, st, t, lt, ovt, ry, [&](int s) { return lcy[s][tl]; }, [&](int s) { return lgb[s][tl]; },
                       rate, ex);
@@ -1702,17 +1735,17 @@ __global__ void __launch_bounds__(BLK) __attribute__((amdgpu_waves_per_eu(4))) k
                         rate);
       });
     } else {
-      __shared__ float lcy[NS + 1][BLK];
-      __shared__ double lgb[NS + 1][BLK];
+      __shared__ float lcy[rows_c<NS, float>][BLK];
+      __shared__ double lgb[rows_g<NS, float>][BLK];
       const int tl = threadIdx.x;
-      lcy[NS][tl] = 1;   // what the lists are filled up with
-      lgb[NS][tl] = 0;
+      if constexpr (rows_c<NS, float> > NS) lcy[NS][tl] = 1;
+      if constexpr (rows_g<NS, float> > NS) lgb[NS][tl] = 0;
 #pragma unroll
       for (int s = 0; s < NS; s++) {
         lcy[s][tl] = ryf[s] * tb->ovwf[s];
         lgb[s][tl] = gibbs[s];
       }
-      RtMech<NS> mr{c, tb};
+      RtMech<NS, fill_rows<NS, float>> mr{c, tb};
       for_steps(mr, [&](int st) {
         chem_stepmx<NS>(mr, st, tf, lt, ovt, ryf, [&](int s) { return lcy[s][tl]; }, [&](int s) { return lgb[s][tl]; },
                         rate);
