@@ -164,9 +164,8 @@ inline __host__ __device__ int nface(int ns) { return face_corr(ns) + 5 + ns; }
 // that member's block b - blk0[kind].  A single case is a launch of one member.
 // L_FACE2: both x faces; L_PASSX: the pass with the x derivatives (x with y, or
 // x alone); L_PASSXE: its edge tiles where x is bounded (two launches then,
-// interior and edge tiles); L_PASSY: empty unless y has a pass of its own;
-// L_CROSS: the tiles of the cross-term kernel where they are the larger ones
-enum LaunchKind { L_FACE = 0, L_FACE2, L_POINT, L_PASSX, L_PASSY, L_PASSZ, L_FINAL, L_PASSXE, L_CROSS, L_NKIND };
+// interior and edge tiles); L_PASSY: empty unless y has a pass of its own
+enum LaunchKind { L_FACE = 0, L_FACE2, L_POINT, L_PASSX, L_PASSY, L_PASSZ, L_FINAL, L_PASSXE, L_NKIND };
 
 struct Member {
   Params P;

@@ -2856,22 +2856,26 @@ __global__ void __launch_bounds__(NSCBC_BLK) k_nscbc(const Member *__restrict__ 
 //
 // Between the substages of a step only the cross terms are formed here (CROSS)
 // and go back to the accumulators; the register update moves to the next
-// point kernel (lincom_point).  At 128^3 and 9 species that is 155 us in FP64
-// and 111 us mixed against 294 and 231 us with the update, while the point
-// kernel grows by 50 and 60 us; an RK step takes 6.74 -> 6.42 ms and 4.41 ->
-// 4.18 ms.
+// point kernel (lincom_point).  At 128^3 and 9 species that is 165 us in FP64
+// and 110 us mixed (bounded x; periodic 125 and 80) against 294 and 231 us with
+// the update, while the point kernel grows by 50 and 60 us; an RK step takes
+// 6.74 -> 6.42 ms and 4.41 -> 4.18 ms.
+//
+// A tile twice as deep (16 x 8 x 8, 512 threads) stages a quarter less halo per
+// point and gains nothing by it: the mean launch of a step at 9 species, with
+// tiles of depth 8 and 4, takes 1160 and 1200 us (256^3, bounded, FP64), 183
+// and 184 (128^3), 63 and 61 (80x80x96), 78 and 70 (81x83x90); mixed 863 and
+// 825, 134 and 124, 51 and 44, 63 and 54.
 //
 // A block owns an FX x FY x FZ tile of points, NPT per thread along z.  The
 // six mixed derivatives (d2u/dxdy, d2u/dxdz, d2v/dxdy, d2v/dydz, d2w/dxdz,
 // d2w/dydz) read their diagonal neighbours from u, v and w staged one at a
 // time into an LDS tile with a 5-deep halo in every direction (wrapped where
 // periodic, clamped where bounded), instead of 120 neighbour loads per point.
-template <bool BIG>
 struct FinalTile {
-  static constexpr int FX = 16, FY = 8, FZ = BIG ? 8 : 4;
-  static constexpr int NT = BIG ? 512 : 256;       // threads
-  static constexpr int NPT = FX * FY * FZ / NT;    // points per thread
-  static constexpr int ZS = NT / (FX * FY);        // z stride between a thread's points
+  static constexpr int FX = 16, FY = 8, FZ = 4;
+  static constexpr int NPT = FX * FY * FZ / BLK;   // points per thread
+  static constexpr int ZS = BLK / (FX * FY);       // z stride between a thread's points
   static constexpr int GX = FX + 10, GY = FY + 10, GZ = FZ + 10, GN = GX * GY * GZ;
 };
 
@@ -3063,14 +3067,13 @@ __device__ __forceinline__ void final_point(const Params &P, const Fields &F, co
   }
 }
 
-template <bool BND, int NS, class R, bool CROSS, bool BIG>
-__global__ void __launch_bounds__(FinalTile<BIG>::NT) __attribute__((amdgpu_waves_per_eu(BIG ? 4 : 1))) k_final(
-    const Member *__restrict__ mem, const uint32_t *__restrict__ map, const sg_config *__restrict__ c, int irk,
-    double *__restrict__ out) {
-  using FT = FinalTile<BIG>;
-  constexpr int FX = FT::FX, FY = FT::FY, FZ = FT::FZ, NPT = FT::NPT, GX = FT::GX, GY = FT::GY;
+template <bool BND, int NS, class R, bool CROSS>
+__global__ void __launch_bounds__(BLK) k_final(const Member *__restrict__ mem, const uint32_t *__restrict__ map,
+                                               const sg_config *__restrict__ c, int irk, double *__restrict__ out) {
+  using FT = FinalTile;
+  constexpr int FX = FT::FX, FY = FT::FY, FZ = FT::FZ, NPT = FT::NPT, GX = FT::GX, GY = FT::GY, GZ = FT::GZ;
   int lb;
-  const Member &M = member_at<BIG ? L_CROSS : L_FINAL>(mem, map, xcd_block(blockIdx.x, gridDim.x), lb);
+  const Member &M = member_at<L_FINAL>(mem, map, xcd_block(blockIdx.x, gridDim.x), lb);
   const Params P = M.P;
   const Fields F = global_fields(M.F);
   // substage irk: LINCOM (mode 0) or FINCOM at the last substage (mode 1);
@@ -3117,18 +3120,18 @@ __global__ void __launch_bounds__(FinalTile<BIG>::NT) __attribute__((amdgpu_wave
     return g < n ? g : n - 1;
   };
   // staging: the tile is GX*GY columns of GZ values; thread t fetches
-  // columns t, t + NT, all loads in flight at once, into registers and then
+  // columns t, t + BLK, all loads in flight at once, into registers and then
   // stores them to LDS.  The next field's fetch is issued before the current
   // field's derivatives are evaluated.  Column offsets are per thread, plane
   // offsets are uniform.  Only what the field's stencils read is fetched: u
   // the (x, y) and (x, z) planes of its points, v (x, y) and (y, z), w (x, z)
   // and (y, z).
-  constexpr int NCOL = GX * GY, GZ = FT::GZ, NTH = FT::NT, NC = (NCOL + NTH - 1) / NTH;
+  constexpr int NCOL = GX * GY, NC = (NCOL + BLK - 1) / BLK;
   uint32_t co[NC];
   bool inx[NC], iny[NC];
 #pragma unroll
   for (int q = 0; q < NC; q++) {
-    const int cc = t + q * NTH, tx = cc % GX, ty = cc / GX;
+    const int cc = t + q * BLK, tx = cc % GX, ty = cc / GX;
     const bool ok = cc < NCOL;
     inx[q] = ok && tx >= 5 && tx < 5 + FX;
     iny[q] = ok && ty >= 5 && ty < 5 + FY;
@@ -3140,7 +3143,7 @@ __global__ void __launch_bounds__(FinalTile<BIG>::NT) __attribute__((amdgpu_wave
 #pragma unroll
     for (int q = 0; q < NC; q++) {
       const bool halo = FLD == 0 ? iny[q] : (FLD == 1 ? inx[q] : inx[q] || iny[q]);   // z halo
-      const bool in = FLD == 2 ? halo : t + q * NTH < NCOL;
+      const bool in = FLD == 2 ? halo : t + q * BLK < NCOL;
       if (in) {
 #pragma unroll
         for (int z = 5; z < 5 + FZ; z++) f(q, z);
@@ -3162,7 +3165,7 @@ __global__ void __launch_bounds__(FinalTile<BIG>::NT) __attribute__((amdgpu_wave
     });
   };
   auto store = [&](auto field) {
-    columns(field, [&](int q, int z) { tile[z * NCOL + t + q * NTH] = stg[q][z]; });
+    columns(field, [&](int q, int z) { tile[z * NCOL + t + q * BLK] = stg[q][z]; });
   };
   using FU = std::integral_constant<int, 0>;
   using FV = std::integral_constant<int, 1>;
@@ -3389,29 +3392,25 @@ void launch_radn_t(const Launch &L, hipStream_t st) {
   if (L.precision) hipLaunchKernelGGL((k_radn<NS, float>), g, b, 0, st, L.mem, L.map[L_POINT], L.c);
   else hipLaunchKernelGGL((k_radn<NS, double>), g, b, 0, st, L.mem, L.map[L_POINT], L.c);
 }
-template <int NS, bool CROSS, bool BIG>
+template <int NS, bool CROSS>
 static void launch_final_c(const Launch &L, int irk, double *out, hipStream_t st) {
-  constexpr int K = BIG ? L_CROSS : L_FINAL;
-  const dim3 g(L.nblk[K]), b(FinalTile<BIG>::NT);
-  const uint32_t *map = L.map[K];
+  const dim3 g(L.nblk[L_FINAL]), b(BLK);
+  const uint32_t *map = L.map[L_FINAL];
   if (L.precision) {
-    if (L.bndx) hipLaunchKernelGGL((k_final<true, NS, float, CROSS, BIG>), g, b, 0, st, L.mem, map, L.c, irk, out);
-    else hipLaunchKernelGGL((k_final<false, NS, float, CROSS, BIG>), g, b, 0, st, L.mem, map, L.c, irk, out);
+    if (L.bndx) hipLaunchKernelGGL((k_final<true, NS, float, CROSS>), g, b, 0, st, L.mem, map, L.c, irk, out);
+    else hipLaunchKernelGGL((k_final<false, NS, float, CROSS>), g, b, 0, st, L.mem, map, L.c, irk, out);
   } else {
-    if (L.bndx) hipLaunchKernelGGL((k_final<true, NS, double, CROSS, BIG>), g, b, 0, st, L.mem, map, L.c, irk, out);
-    else hipLaunchKernelGGL((k_final<false, NS, double, CROSS, BIG>), g, b, 0, st, L.mem, map, L.c, irk, out);
+    if (L.bndx) hipLaunchKernelGGL((k_final<true, NS, double, CROSS>), g, b, 0, st, L.mem, map, L.c, irk, out);
+    else hipLaunchKernelGGL((k_final<false, NS, double, CROSS>), g, b, 0, st, L.mem, map, L.c, irk, out);
   }
 }
 template <int NS>
 void launch_final_t(const Launch &L, int irk, double *out, hipStream_t st) {
-  launch_final_c<NS, false, false>(L, irk, out, st);
+  launch_final_c<NS, false>(L, irk, out, st);
 }
-// 16 x 8 x 8 tiles (half the halo of 16 x 8 x 4) once they fill the chip's 512
-// block slots; below that the smaller tiles finish earlier
 template <int NS>
 void launch_cross_t(const Launch &L, hipStream_t st) {
-  if (L.nblk[L_CROSS] >= 512) launch_final_c<NS, true, true>(L, 0, nullptr, st);
-  else launch_final_c<NS, true, false>(L, 0, nullptr, st);
+  launch_final_c<NS, true>(L, 0, nullptr, st);
 }
 
 #ifdef SG_NS
@@ -3468,8 +3467,7 @@ void member_blocks(const Params &P, int nblk[L_NKIND]) {
   auto tiles = [&](int tx, int ty, int tz) {
     return ((P.nx + tx - 1) / tx) * ((P.ny + ty - 1) / ty) * ((P.nz + tz - 1) / tz);
   };
-  nblk[L_FINAL] = tiles(FinalTile<false>::FX, FinalTile<false>::FY, FinalTile<false>::FZ);
-  nblk[L_CROSS] = tiles(FinalTile<true>::FX, FinalTile<true>::FY, FinalTile<true>::FZ);
+  nblk[L_FINAL] = tiles(FinalTile::FX, FinalTile::FY, FinalTile::FZ);
   // passes: every tile of a row (periodic x), or the interior tiles of the
   // bounded rows (L_PASSX) and their edge tiles (L_PASSXE); y goes with x
   // where the launch has no transport options

@@ -55,3 +55,11 @@ def test_fill_up_rows_cost_no_block(kernels, ns):
         want = min(4, LDS // (ns * BLK * (size + 8) + extra))
         for k in _get(kernels, kernel):
             assert min(4, LDS // k["group_segment_fixed_size"]) == want, (kernel, k["group_segment_fixed_size"])
+
+
+def test_cross_kernels_do_not_spill(kernels):
+    """k_final<BND, NS, R, true>: every form between the substages keeps its
+    three fields' derivatives in registers."""
+    got = _get(kernels, r"_ZN2sg7k_finalILb[01]ELi\d+E[df]Lb1E")
+    assert len(got) >= 2 * 2 * 17
+    assert [k["vgpr_spill_count"] for k in got if k["vgpr_spill_count"]] == []
