@@ -65,29 +65,33 @@ def copy_calibration(h, nbytes=1 << 30):
     print(f"copy calibration: {nbytes} bytes device-to-device", file=sys.stderr, flush=True)
 
 
-def kernel_bytes(name, ns, bounded, nx=128):
+def kernel_bytes(name, ns, bounded, nx=128, prec="fp64"):
     """Algorithmic bytes per grid point of one launch: each distinct input
-    field read once and each output written once (FP64 fields, 4-byte index).
-    The face kernels touch the nx = 1 and nx = n planes only: their bytes are
-    spread over the grid (divided by nx).  prim and final: the mean over the
-    five launches of a step, of which four of prim begin with the register
-    update and four of final only add the cross terms."""
-    f = 8
+    field read once and each output written once.  FP64: the two registers and
+    the face arrays, and in the FP64 form every field; the mixed form (prec
+    "mixed") holds primitives, rates, accumulators and gradients in FP32; the
+    interval index has 4 bytes.  The face kernels touch the nx = 1 and nx = n
+    planes only: their bytes are spread over the grid (divided by nx).  prim
+    and final: the mean over the five launches of a step, of which four of prim
+    begin with the register update and four of final only add the cross terms."""
+    f, w = 8, 4 if prec == "mixed" else 8
+    reg = f * (5 + ns)
+    acc = w * (5 + ns)
     nprim = 9 + 3 * ns
     if name in ("boundt", "bountt"):   # inflow values of 5+N fields at x-left
-        return f * (5 + ns) / nx
+        return reg / nx
     if name == "nscbc":                # face data (6+N) + stage register (5+N) + corrections (5+N), two faces
-        return 2 * f * ((6 + ns) + 2 * (5 + ns)) / nx
+        return 2 * (f * (6 + ns) + 2 * reg) / nx
     if name == "prim":          # reads stage (5+N), T, index; writes primitives, rate, index;
-        io = f + 4 + f * (nprim + ns) + 4   # after an update: accumulators, run (r/w), 4 stage fields (w) for the stage
-        return (f * (5 + ns) + io + 4 * (3 * f * (5 + ns) + 4 * f + io)) / 5
-    if name == "pass_x":        # x with y: rho, 3 momenta, primitives, rate -> accumulators, d mu/dx, d mu/dy
-        return f * (4 + nprim + ns) + f * (5 + ns) + 2 * f
-    if name in ("pass_y", "pass_z"):   # accumulators read-modify-write
-        return f * (4 + nprim) + 2 * f * (5 + ns) + f
+        io = w + 4 + w * (nprim + ns) + 4   # after an update: accumulators, run (r/w), 4 stage fields (w) for the stage
+        return (reg + io + 4 * (acc + 2 * reg + 4 * f + io)) / 5
+    if name == "pass_x":        # x with y: 2 momenta, primitives, rate -> accumulators, d mu/dx, d mu/dy
+        return f * 2 + w * (nprim + ns) + acc + 2 * w
+    if name in ("pass_y", "pass_z"):   # 1 momentum, primitives, accumulators read-modify-write, d mu
+        return f + w * nprim + 2 * acc + w
     if name == "final":         # 3 viscosity gradients, u,v,w,mu; accumulators, run (r/w), stage (w), or
-        io = f * 3 + f * 4      # momentum and energy accumulators (r/w)
-        return (io + f * (5 + ns) + 2 * f * (5 + ns) + f * (5 + ns) + 4 * (io + 8 * f)) / 5
+        io = w * 3 + w * 4      # momentum and energy accumulators (r/w)
+        return (io + acc + 2 * reg + reg + 4 * (io + 8 * w)) / 5
     return 0
 
 
@@ -117,7 +121,7 @@ def kernel_table(kern, ns, npts, n, prec):
     out = {}
     for k, (tot, cnt) in kern.items():
         ms = tot / cnt
-        ab = kernel_bytes(k, ns, True, n)
+        ab = kernel_bytes(k, ns, True, n, prec)
         e = {"ms": ms, "algorithmic_bytes_per_point": ab,
              "hbm_achieved_gbs": ab * npts / (ms / 1e3) / 1e9,
              "hbm_frac": ab * npts / (ms / 1e3) / HBM_PEAK}
