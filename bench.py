@@ -231,7 +231,7 @@ def mixed_run(abi, c, a, h, s64):
     s = abi.Solver(c, precision=1)
     s.set_timestep(c.dump.tstep)
     s.upload(c.dump.state, 0.0)
-    tuned = (s.tiles(), None) if a.no_autotune else s.autotune(5)
+    passes_ms = None if a.no_autotune else s.autotune(5)[1]
     stream = C.c_void_p(s.stream())
     ev0, ev1 = C.c_void_p(), C.c_void_p()
     h.hipEventCreate(C.byref(ev0))
@@ -266,7 +266,7 @@ def mixed_run(abi, c, a, h, s64):
             "max_rel_err_T": rel(T32, T64), "max_rel_err_Y": max(rel(r32[5 + k], r64[5 + k]) for k in range(ns)),
             "max_rel_err_conserved": max(rel(r32[v], r64[v]) for v in range(5 + ns)),
             "steps_compared": a.warmup + a.steps + a.profile_steps,
-            "tiles": {"narrow_pass_tiles": list(tuned[0]), "autotuned": not a.no_autotune},
+            "passes_ms_per_substage": passes_ms,
             "kernel_ms_per_launch": {k: round(v[0] / v[1], 4) for k, v in prof.items() if v[1] > 0},
             "kernels": kernel_table({k: v for k, v in prof.items() if v[1] > 0 and kernel_bytes(k, ns, True, c.shape[0]) > 0},
                                     ns, n3, c.shape[0], "mixed")}
@@ -274,7 +274,7 @@ def mixed_run(abi, c, a, h, s64):
 
 def large_run(abi, h, c, steps, warmup=2):
     """FP64 and mixed throughput on a larger grid of the same physics (state
-    resident, tiles autotuned), timed with events on the library's stream."""
+    resident), timed with events on the library's stream."""
     n3 = c.shape[0] * c.shape[1] * c.shape[2]
     out = {"grid": list(c.shape), "steps": steps}
     ev0, ev1 = C.c_void_p(), C.c_void_p()
@@ -284,7 +284,6 @@ def large_run(abi, h, c, steps, warmup=2):
         s = abi.Solver(c, precision=prec)
         s.set_timestep(c.dump.tstep)
         s.upload(c.dump.state, 0.0)
-        tiles, _ = s.autotune(3)
         s.step(warmup)
         s.sync()
         stream = C.c_void_p(s.stream())
@@ -296,8 +295,7 @@ def large_run(abi, h, c, steps, warmup=2):
         ms = C.c_float(0)
         h.hipEventElapsedTime(C.byref(ms), ev0, ev1)
         out[tag] = {"value": round(n3 * 5 * steps / (ms.value / 1e3) / 1e6, 3), "unit": "Mpoint-RK-substages/s",
-                    "ms_per_step": round(ms.value / steps, 4), "device_bytes": s.memory(),
-                    "narrow_pass_tiles": list(tiles)}
+                    "ms_per_step": round(ms.value / steps, 4), "device_bytes": s.memory()}
         s.close()
         print(f"{c.shape} {tag}: {ms.value:.2f} ms for {steps} steps", file=sys.stderr, flush=True)
     out["speedup_mixed"] = out["mixed"]["value"] / out["fp64"]["value"]
@@ -338,10 +336,9 @@ def batched_run(abi, h, cases, steps):
             s.set_timestep(c.dump.tstep)
             s.upload(c.dump.state, 0.0)
             sols.append(s)
-        # sequential: each case on its own (tiles autotuned per case), one after the other
+        # sequential: each case on its own, one after the other
         if prec == 0:
             for s in sols:
-                s.autotune(3)
                 s.step(1)
             h.hipDeviceSynchronize()
             t0 = time.perf_counter()
@@ -352,7 +349,6 @@ def batched_run(abi, h, cases, steps):
         b = abi.Batch()
         for s in sols:
             b.add(s)
-        tiles, _ = b.autotune(3)
         b.step(1)
         b.sync()
         t0 = time.perf_counter()
@@ -361,7 +357,7 @@ def batched_run(abi, h, cases, steps):
         t_b = time.perf_counter() - t0
         tag = "fp64" if prec == 0 else "mixed"
         out[tag] = {"cases_per_s": len(cases) / (t_b * 100.0 / steps), "s_per_step": t_b / steps,
-                    "mpoint_substages_per_s": pts * 5 * steps / t_b / 1e6, "autotuned_narrow_tiles": list(tiles)}
+                    "mpoint_substages_per_s": pts * 5 * steps / t_b / 1e6}
         if prec == 0:
             out["sequential_fp64"] = {"cases_per_s": len(cases) / (t_seq * 100.0 / steps),
                                       "s_per_step": t_seq / steps,
@@ -485,7 +481,7 @@ def main():
                     help="grid of the second FP64/mixed throughput figure (0: skip)")
     ap.add_argument("--large-steps", type=int, default=5)
     ap.add_argument("--no-autotune", action="store_true",
-                    help="keep the default tiles (profiling runs: no tuning launches in the trace)")
+                    help="do not time the passes apart (profiling runs: none of their launches in the trace)")
     ap.add_argument("--study-steps", type=int, default=0,
                     help="instead of the throughput run: FP64 vs mixed on the --n case for this many "
                          "steps, per-field errors")
@@ -528,8 +524,7 @@ def main():
     s = abi.Solver(c)
     s.set_timestep(c.dump.tstep)
     s.upload(c.dump.state, 0.0)
-    tuned = (s.tiles(), None) if a.no_autotune else s.autotune(5)
-    print(f"tiles {tuned}", file=sys.stderr, flush=True)
+    passes_ms = None if a.no_autotune else s.autotune(5)[1]
     h = hip()
     if a.copy_calibration:
         copy_calibration(h)
@@ -603,7 +598,7 @@ def main():
         "substage": substage,
         "kernels": table,
         "kernel_ms_per_launch": {k: round(v["ms"], 4) for k, v in table.items()},
-        "tiles": {"narrow_pass_tiles": list(tuned[0]), "autotuned": not a.no_autotune},
+        "passes_ms_per_substage": passes_ms,
     }
     if not a.no_mixed:
         out["mixed"] = mixed_run(abi, c, a, h, s)
@@ -611,7 +606,7 @@ def main():
     if lcases:
         out["large"] = large_run(abi, h, lcases[0], a.large_steps)
         out["large"]["workload"] = (f"the same H2-air NSCBC physics on {a.large_n}^3 (grid spacing of the 128^3 "
-                                    f"/ 5 mm case), {a.large_steps} RK steps timed after 2, tiles autotuned")
+                                    f"/ 5 mm case), {a.large_steps} RK steps timed after 2")
     if bcases:
         out["batched"] = batched_run(abi, h, bcases, a.batch_steps)
         out["batched"]["workload"] = (f"{len(bcases)} H2-air NSCBC cases, n^3 with n from {{48,64,96,128}}, "

@@ -285,13 +285,13 @@ int sg_memory(sg_handle *h, size_t *bytes);
  * counterpart in the reference, which reads chem.dat at run time. */
 int sg_mechanism_compiled(const sg_handle *h, int *compiled);
 
-/* ---- Tiles and their autotuner (no counterpart in the reference) ---------
+/* ---- Tile flags and timing of the passes (no counterpart in the reference)
  * The derivative passes have one tile shape (16 x 16 points, see k_pass), so
  * there is nothing left to choose: narrow[d] (0 or 1, kept for callers that
  * set it) is stored and returned and changes neither results nor speed.
  * sg_autotune times the passes on the handle's current state (reps launches
  * each, 5 if reps <= 0) and returns in *ms their time per substage; the state
- * it leaves is the one it found, so tuned and untuned runs compute identical
+ * it leaves is the one it found, so runs with and without it compute identical
  * results. */
 int sg_set_tiles(sg_handle *h, const int narrow[3]);
 int sg_get_tiles(sg_handle *h, int narrow[3]);

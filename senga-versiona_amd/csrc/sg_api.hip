@@ -1314,7 +1314,8 @@ int sg_batch_member(sg_batch *b, int idx, sg_handle **h) {
 // A timing run launches the passes on the live state.  It changes nothing a later
 // step reads except the stored temperature (the Newton initial guess) and the
 // interval indices, which prim rewrites; those are saved and put back, so a
-// tuned run computes exactly what an untuned one does.
+// run with it computes exactly what one without it does.  Member records and
+// block maps stay, and with them a batch's captured step.
 struct TempSnap {
   void *buf = nullptr;
   size_t tb = 0, ib = 0;
@@ -1398,7 +1399,6 @@ int sg_autotune(sg_handle *h, int reps, double *ms) {
   double total = 0.0;
   for (int d = 0; d < 3; d++) total += time_launches(h->stream, reps, [&] { launch_pass(d, h->L, h->stream); });
   rc = snap_restore(h, sn, h->stream);
-  if (!rc) rc = refresh_member(h);
   if (!rc && ms) *ms = total;
   return rc;
 }
@@ -1419,7 +1419,6 @@ int sg_batch_autotune(sg_batch *b, int reps, double *ms) {
   if (!b) return SG_EINVAL;
   if (b->members.empty()) return 0;
   if (reps <= 0) reps = 5;
-  b->dirty_layout = 1;
   int rc = batch_prepare(b);
   if (rc) return rc;
   std::vector<TempSnap> sn(b->members.size());

@@ -2861,8 +2861,8 @@ __global__ void __launch_bounds__(NSCBC_BLK) k_nscbc(const Member *__restrict__ 
 // the update, while the point kernel grows by 50 and 60 us; an RK step takes
 // 6.74 -> 6.42 ms and 4.41 -> 4.18 ms.
 //
-// A tile twice as deep (16 x 8 x 8, 512 threads) stages a quarter less halo per
-// point and gains nothing by it: the mean launch of a step at 9 species, with
+// A tile twice as deep (16 x 8 x 8, 512 threads) stages 19 values a point instead
+// of 27 and gains nothing by it: the mean launch of a step at 9 species, with
 // tiles of depth 8 and 4, takes 1160 and 1200 us (256^3, bounded, FP64), 183
 // and 184 (128^3), 63 and 61 (80x80x96), 78 and 70 (81x83x90); mixed 863 and
 // 825, 134 and 124, 51 and 44, 63 and 54.
