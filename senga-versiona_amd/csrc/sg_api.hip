@@ -411,6 +411,7 @@ static int setup_params(sg_handle *h) {
   P.pofs = c.precision ? c.prin : 0.0;
   P.alamda = c.alamda; P.rlamda = c.rlamda; P.prantl = c.prantl;
   P.tdifgb = c.tdifgb; P.pdifgb = c.pdifgb;
+  P.xsplit = pass_split(P);
   return 0;
 }
 

@@ -26,6 +26,7 @@ struct Params {
   long npts;                   // nx*ny*nz
   long fstride;                // elements between consecutive fields
   int bnd[3];                  // 1: direction bounded (closures), 0: periodic
+  int xsplit;                  // bounded x: the passes' rows in edge and interior tiles (pass_split)
   double ovdel[3], ovdl2[3];
   double ac[5], c1[4], c2[4], c3[2], c4[3], c5[4];       // first derivative
   double sc[5], s1[5], s2[5], s3[2], s4[3], s5[4];       // second derivative
@@ -194,6 +195,36 @@ struct Launch {
 // Whether the x and y derivatives are formed in one pass: without the
 // molecular-transport options.
 inline bool pass_xy(const Params &P) { return !(P.mixw || P.mixp || P.soret || P.dufour); }
+
+// Tiles of the passes along a row (16 points each).  A bounded row is split,
+// an edge tile at either end and interior tiles between them (two launches),
+// on grids of more tiles than the chip holds blocks at two waves a SIMD; below
+// that every tile is an edge tile and the pass one launch.  An edge tile costs
+// half as much again as an interior one, but two launches of a part-filled
+// chip take twice the time of one: a step at 9 species, FP64, split and not,
+// takes 549 and 466 us at 40x24x24 (144 tiles of 512 places), 628 and 555 at
+// 48^3 (432), 889 and 888 at 64^3 (1024), 1729 and 1801 at 128x64x64 (2048); 2
+// species mixed 349 and 287, 414 and 352, 454 and 387, 632 and 620; 16 species
+// with all options 1135 and 1022 at 64x32x32 (256 of 256), 1285 and 1299 at
+// 48x40x40 (360).  Of a batch each member goes by its own size, so that it
+// computes what it computes alone: 32 members of 33^3 to 47^3 take 8.28 ms a
+// step split and 7.94 not.
+constexpr int PASS_EW = 16;
+constexpr int pass_waves(int ns) { return 1 + (ns + 2) / 3; }   // of a block of a pass with x derivatives
+inline int pass_split(const Params &P) {
+  if (!P.bnd[0] || P.nx < 2 * PASS_EW) return 0;
+  const long tiles = (long)((P.nx + 15) / 16) * ((P.ny + 15) / 16) * P.nz;
+  return tiles > 256L * (8 / pass_waves(P.ns));
+}
+inline __host__ __device__ int pass_xtiles(const Params &P, int xp) {
+  if (xp == 1) return P.xsplit ? (P.nx - 2 * PASS_EW + 15) / 16 : 0;
+  return xp == 2 && P.xsplit ? 2 : (P.nx + 15) / 16;
+}
+// first x index of x tile bx
+inline __host__ __device__ int pass_x0(const Params &P, int xp, int bx) {
+  if (xp == 1) return PASS_EW + bx * 16;
+  return xp == 2 && P.xsplit ? (bx == 0 ? 0 : P.nx - PASS_EW) : bx * 16;
+}
 
 // member block counts of each kind (sg_kernels.hip)
 void member_blocks(const Params &P, int nblk[L_NKIND]);

@@ -1902,26 +1902,14 @@ __global__ void __launch_bounds__(BLK) __attribute__((amdgpu_waves_per_eu(4))) k
 // Products with rho u_d (e rho u_d, Y rho u_d and the momentum fluxes rho u_d
 // u_b) are formed inside the stencils from two tiles.
 //
-// Bounded x direction: x passes run as two launches.  Edge tiles, PASS_EW
-// points wide at each end of a row, hold every closure row (i < 5, i > nx - 6)
-// and evaluate their x stencils with per-column weights; interior tiles
-// cover [PASS_EW, nx - PASS_EW), where every stencil is the interior one and
-// reaches no further than 5 points into the edge tiles.  xp: 0 every x tile
-// of a row (periodic x, and the y and z passes); 1 the interior tiles of a
-// bounded row; 2 its edge tiles.  Rows shorter than 2 PASS_EW are all edge
-// tiles.
-constexpr int PASS_EW = 16;
-__host__ __device__ inline int pass_xtiles(int nx, int xp, int tx) {
-  if (xp == 0) return (nx + tx - 1) / tx;
-  if (xp == 1) return nx >= 2 * PASS_EW ? (nx - 2 * PASS_EW + tx - 1) / tx : 0;
-  return nx >= 2 * PASS_EW ? 2 : (nx + PASS_EW - 1) / PASS_EW;
-}
-// first x index of x tile bx
-__host__ __device__ inline int pass_x0(int nx, int xp, int tx, int bx) {
-  if (xp == 0) return bx * tx;
-  if (xp == 1) return PASS_EW + bx * tx;
-  return nx >= 2 * PASS_EW ? (bx == 0 ? 0 : nx - PASS_EW) : bx * PASS_EW;
-}
+// Bounded x direction (pass_xtiles): rows of large grids are split in two
+// launches.  Edge tiles at each end of a row hold every closure row (i < 5,
+// i > nx - 6) and evaluate their x stencils with per-column weights; interior
+// tiles between them take the interior stencil everywhere and reach no further
+// than 5 points into the edge tiles.  Grids whose tiles fit the chip at once
+// take edge tiles all along the row, in one launch.  xp: 0 every x tile of a
+// row (periodic x, and the y and z passes); 1 the interior tiles of a bounded
+// row; 2 its edge tiles.
 
 // The block of a pass: a tile of 16 x-points times 16 rows along y (or along
 // z, DV = 2), worked by one wave for the hydrodynamic fields and one wave per
@@ -1941,6 +1929,7 @@ struct PassTile {
   static constexpr int NG = (NS + SPMAX - 1) / SPMAX;      // species waves
   static constexpr int SPW = (NS + NG - 1) / NG;
   static constexpr int NW = 1 + NG, NT = 64 * NW;
+  static_assert(!DX || NW == pass_waves(NS), "the wave count pass_split assumes");
   // LDS tile: rows padded so that the four rows a wave reads at once (4 apart)
   // start on different banks
   static constexpr int LXU = T + 2 * HX, LV = T + 2 * HV;
@@ -1994,7 +1983,7 @@ __attribute__((amdgpu_waves_per_eu(sizeof(R) == 8 ? 2 : (DX + (DV != 0) == 2 ? 3
   const Fields F = global_fields(M.F);
   // tile origin: x0, and row v0 along y (z for DV = 2) in plane w0
   const int nv = DV == 2 ? P.nz : P.ny, nw = DV == 2 ? P.ny : P.nz;
-  const int nbx = pass_xtiles(P.nx, XP, T), nbv = (nv + T - 1) / T;
+  const int nbx = pass_xtiles(P, XP), nbv = (nv + T - 1) / T;
   int bv, w0;
   if (DV == 2) {   // planes before rows of tiles, so that x rows of one z follow each other
     w0 = (lb / nbx) % nw;
@@ -2003,7 +1992,7 @@ __attribute__((amdgpu_waves_per_eu(sizeof(R) == 8 ? 2 : (DX + (DV != 0) == 2 ? 3
     bv = (lb / nbx) % nbv;
     w0 = lb / (nbx * nbv);
   }
-  const int x0 = pass_x0(P.nx, XP, T, lb % nbx), v0 = bv * T;
+  const int x0 = pass_x0(P, XP, lb % nbx), v0 = bv * T;
   // this lane's points: column x, rows 4 q .. 4 q + 3 of the tile
   const int lx = lane & 15, q4 = (lane >> 4) * 4;
   const int i = x0 + lx;
@@ -3468,12 +3457,12 @@ void member_blocks(const Params &P, int nblk[L_NKIND]) {
     return ((P.nx + tx - 1) / tx) * ((P.ny + ty - 1) / ty) * ((P.nz + tz - 1) / tz);
   };
   nblk[L_FINAL] = tiles(FinalTile::FX, FinalTile::FY, FinalTile::FZ);
-  // passes: every tile of a row (periodic x), or the interior tiles of the
-  // bounded rows (L_PASSX) and their edge tiles (L_PASSXE); y goes with x
-  // where the launch has no transport options
+  // passes: every tile of a row (periodic x), or of bounded rows the interior
+  // tiles (L_PASSX) and the edge tiles (L_PASSXE); y goes with x where the
+  // launch has no transport options
   const long rows = (long)((P.ny + 15) / 16) * P.nz;
-  nblk[L_PASSX] = (int)(pass_xtiles(P.nx, P.bnd[0] ? 1 : 0, 16) * rows);
-  nblk[L_PASSXE] = P.bnd[0] ? (int)(pass_xtiles(P.nx, 2, 16) * rows) : 0;
+  nblk[L_PASSX] = (int)(pass_xtiles(P, P.bnd[0] ? 1 : 0) * rows);
+  nblk[L_PASSXE] = P.bnd[0] ? (int)(pass_xtiles(P, 2) * rows) : 0;
   nblk[L_PASSY] = pass_xy(P) ? 0 : tiles(16, 16, 1);
   nblk[L_PASSZ] = tiles(16, 1, 16);
 }
