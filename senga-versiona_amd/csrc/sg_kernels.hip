@@ -1961,8 +1961,11 @@ struct PassTile {
 
 // Registers: an FP64 wave holds its species' right-hand sides and gradients
 // of four points per lane (36 values with two directions) beside a 14-value
-// stencil window, which takes the 256 registers of two waves per SIMD (254 in
-// the x-y pass, 214-228 in z); FP32 fits three (x with y) and four waves.
+// stencil window, which takes the 256 registers of two waves per SIMD: 224 in z
+// at 9 species, all and 6 to 9 spilled in the x-y pass (18 to 26 where 5, 7 or
+// 8 species make uneven waves, up to 46 at 10 to 12 and 93 at 16 to 18, where
+// it is still faster than x and y apart: 153 against 105 + 72 us at 64^3 and 16
+// species); FP32 fits three (x with y) and four waves.
 // With one spill per lane and field the z pass was 40% slower, hence the sums
 // kept in LDS and the branches that end in a barrier of their own.
 template <int DX, int DV, bool BND, int NS, class R, int XP = 0, bool EXT = false>
@@ -2845,9 +2848,9 @@ __global__ void __launch_bounds__(NSCBC_BLK) k_nscbc(const Member *__restrict__ 
 //
 // Between the substages of a step only the cross terms are formed here (CROSS)
 // and go back to the accumulators; the register update moves to the next
-// point kernel (lincom_point).  At 128^3 and 9 species that is 165 us in FP64
-// and 110 us mixed (bounded x; periodic 125 and 80) against 294 and 231 us with
-// the update, while the point kernel grows by 50 and 60 us; an RK step takes
+// point kernel (lincom_point).  At 128^3 and 9 species that is 154 us in FP64
+// and 97 us mixed (bounded x; periodic about a fifth less) against 294 and 231
+// us with the update, while the point kernel grows by 50 and 60 us; an RK step takes
 // 6.74 -> 6.42 ms and 4.41 -> 4.18 ms.
 //
 // A tile twice as deep (16 x 8 x 8, 512 threads) stages 19 values a point instead
